@@ -325,7 +325,8 @@ LLMIK_API void llmik_w4a16_set_plan_override(int stream_mode, int stream_splits)
  * path with 16-token tiles, 0 with 32-token tiles, -1 restores the rule (16-
  * token tiles for at least 32 (batch, kv head, head chunk) slabs, a
  * workgroup count that is a multiple of the CU count, and at least two
- * 32-token tiles per wave unless the workgroups have 4 waves). Not
+ * 32-token tiles per wave unless the workgroups have 4 waves or 8 query
+ * heads; chunks of 3 query heads never take them). Not
  * synchronised with calls in flight on other threads.
  */
 LLMIK_API void llmik_attention_set_plan_override(int f16_half_tiles);

@@ -6,8 +6,9 @@
 // with the cache addressed at stride kv_buf_len and read over [0, seqlen).
 //
 // Work decomposition (both kernels below)
-//   * One workgroup owns one (batch, kv_head, head_chunk, split): the
-//     HPW <= 4 query heads that share a kv head are processed together, so
+//   * One workgroup owns one (batch, kv_head, head_chunk, split): up to 8
+//     query heads that share a kv head (HPW, the power of two that holds
+//     them) are processed together, so with up to 8 query heads per kv head
 //     every K/V byte of the split is read from HBM exactly once (the
 //     reference re-reads each kv head once per query head,
 //     kernels/attention/fused_attention_splitk.cu:84-90).
@@ -19,10 +20,11 @@
 //
 // Main kernel (decode_attention_mfma_kernel): each wave walks its tiles of
 // 32 tokens on v_mfma_f32_16x16x32_f16:
-//   QK : A = q (16 rows, row m holds head (m / 4) % HPW), B = 16 tokens'
-//        keys (lane = token, 8 consecutive channels per lane group) -> lane
-//        group g gets head g % HPW's score of its token and runs that head's
-//        online softmax; no cross-group reductions.
+//   QK : A = q (16 rows, row m holds head (m / 4) % HPW; HPW = 8: lane group
+//        g's four rows hold heads g and g + 4), B = 16 tokens' keys (lane =
+//        token, 8 consecutive channels per lane group) -> lane group g gets
+//        its one or two heads' scores of its token and runs their online
+//        softmax; no cross-group reductions.
 //   PV : A = p as an fp16 hi + lo pair (two MFMAs per B operand, through a
 //        512-byte per-wave LDS slot; fp16 p alone would cost ~2^-12 |v| of
 //        accuracy under a peaked softmax), B = values:
@@ -50,6 +52,7 @@
 //   I4 : k,v [B,Hkv,L,64] packed int4 (even channel in the low nibble),
 //        k_scale [B,Hkv,n_groups,128] fp16 (per channel, per group of
 //        group_size tokens), v_scale [B,Hkv,L] fp16 (per token)
+#include <algorithm>
 #include <atomic>
 
 #include "device_common.hpp"
@@ -82,7 +85,21 @@ struct AttnParams {
     int group_size, n_groups;
     int n_splits, chunk, n_hchunks, gqa;
     float scale_log2;
+    int heads_per_chunk;   // query heads of a head chunk (the last one may hold fewer)
 };
+
+// Query heads of head chunk `hchunk`, at most HPW. PAD: the chunks hold fewer
+// heads than HPW; the MFMA kernels then compute HPW heads all the same, the
+// rows past the chunk's heads repeat its last head and are not stored.
+template <int HPW, bool PAD>
+__device__ __forceinline__ int chunk_heads(const AttnParams& p, int hchunk) {
+    return PAD ? min(p.heads_per_chunk, p.gqa - hchunk * p.heads_per_chunk) : HPW;
+}
+// The first query head of head chunk `hchunk` of kv head `kvh`.
+template <int HPW, bool PAD>
+__device__ __forceinline__ int chunk_head0(const AttnParams& p, int kvh, int hchunk) {
+    return kvh * p.gqa + hchunk * (PAD ? p.heads_per_chunk : HPW);
+}
 
 // Split hand-off. Thread t < HPW * 32 of the workgroup owns head t / 32,
 // channels 4 (t % 32) .. + 3 of the workgroup's outputs; the partials and
@@ -150,7 +167,7 @@ __device__ __forceinline__ void combine_splits(const AttnParams& p, int b, int s
 // Shared tail: merge NR partial states held in LDS, then either write the
 // output (single split) or publish the split and let the last one combine.
 // ---------------------------------------------------------------------------
-template <int NR, int HPW, int NT>
+template <int NR, int HPW, int NT, bool PAD>
 __device__ __forceinline__ void finish_split(const AttnParams& p, const float (*s_o)[HPW][kHeadDim],
                                              const float (*s_m)[HPW], const float (*s_l)[HPW],
                                              uint32_t* s_last, int b, int kvh, int hchunk,
@@ -158,7 +175,7 @@ __device__ __forceinline__ void finish_split(const AttnParams& p, const float (*
     constexpr int kThr = HPW * (kHeadDim / 4);   // threads owning four outputs
     static_assert(NT >= kThr, "the workgroup must cover every output");
     const int tid = threadIdx.x;
-    const bool owner = tid < kThr;
+    const bool owner = tid < chunk_heads<HPW, PAD>(p, hchunk) * (kHeadDim / 4);
     const int h = owner ? tid / (kHeadDim / 4) : 0;
     const int d = owner ? 4 * (tid % (kHeadDim / 4)) : 0;
     const int slot_group = (b * p.n_kv_heads + kvh) * p.n_hchunks + hchunk;
@@ -455,7 +472,7 @@ struct MfmaTile<KvFormat::I4> {
 // workgroup's waves finish within a tile of each other. INT4: each wave takes
 // a contiguous quarter / eighth of the split, so its K-scale group changes
 // only every group_size tokens.
-template <KvFormat F, int HPW, int NW>
+template <KvFormat F, int HPW, int NW, bool PAD>
 __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_attention_mfma_kernel(AttnParams p) {
     const int split = blockIdx.x;
@@ -468,11 +485,16 @@ void decode_attention_mfma_kernel(AttnParams p) {
     const int g = lane >> 4;
     const int c = lane & 15;
 
-    const int head0 = kvh * p.gqa + hchunk * HPW;
+    const int head0 = chunk_head0<HPW, PAD>(p, kvh, hchunk);
     // QK's A operand row m holds head (m / 4) % HPW: the four outputs of lane
     // group g (rows 4g..4g+3) are all head g % HPW's scores, so each lane
     // group runs the online softmax of one head (PV keeps row m = head m % HPW).
-    const uint16_t* qrow = p.q + ((long)b * p.n_heads + head0 + ((c >> 2) % HPW)) * kHeadDim;
+    // HPW = 8 (HPL = 2 heads per lane group): rows 4g.. hold heads g and
+    // g + 4, alternating (INT4, whose rows alternate hi and lo: two rows each).
+    constexpr int HPL = HPW > 4 ? 2 : 1;
+    const int nh = chunk_heads<HPW, PAD>(p, hchunk);
+    const int hrow = HPL == 2 ? (c >> 2) + 4 * ((F == KvFormat::I4 ? c >> 1 : c) & 1) : (c >> 2) % HPW;
+    const uint16_t* qrow = p.q + ((long)b * p.n_heads + head0 + (PAD ? min(hrow, nh - 1) : hrow)) * kHeadDim;
 
     // Q as the A operand (4 k-steps). INT4: q * k_scale as an fp16 hi + lo
     // pair, hi in the even and lo in the odd rows of each lane group's four,
@@ -500,8 +522,13 @@ void decode_attention_mfma_kernel(AttnParams p) {
     // once at the end: o_j = (o_j - kVBias * sum_p) * kVUnscale.
     f32x4 sum_p = {0.0f, 0.0f, 0.0f, 0.0f};
     const f16x8 ones = {(f16)1.0f, (f16)1.0f, (f16)1.0f, (f16)1.0f, (f16)1.0f, (f16)1.0f, (f16)1.0f, (f16)1.0f};
-    // Online-softmax state of this lane group's head (the same in its 16 lanes).
-    float m_run = -INFINITY, l_run = 0.0f;
+    // Online-softmax state of this lane group's heads (the same in its 16 lanes).
+    float m_run[HPL], l_run[HPL];
+#pragma unroll
+    for (int i = 0; i < HPL; ++i) {
+        m_run[i] = -INFINITY;
+        l_run[i] = 0.0f;
+    }
 
     // P as an fp16 hi + lo pair (plane 0: fp16(x), plane 1: fp16(x - hi)),
     // so that the PV products carry p to ~2^-22 instead of fp16's 2^-12.
@@ -510,11 +537,14 @@ void decode_attention_mfma_kernel(AttnParams p) {
     // and 2 accumulate the hi products and 1 and 3 the lo products in one
     // MFMA, and the two halves are added once at the end (measured: faster
     // for INT4, whose QK already carries a hi/lo pair; not for fp16 / INT8).
-    constexpr bool kPlaneRows = (F == KvFormat::I4);
-    __shared__ __attribute__((aligned(16))) uint16_t s_p[NW][2][4][kTile];
+    // HPW = 8, every format: row m holds plane m / 8 of head m % 8, so the 16
+    // rows are all used and lane groups 0, 1 (hi) add to 2, 3 (lo).
+    constexpr bool kPlaneRows = (F == KvFormat::I4) || HPL == 2;
+    constexpr int kPHeads = HPL == 2 ? 8 : 4;
+    __shared__ __attribute__((aligned(16))) uint16_t s_p[NW][2][kPHeads][kTile];
     // Each head's rescale factor of the tile, for the PV accumulators, which
-    // hold all heads in every lane.
-    __shared__ __attribute__((aligned(16))) float s_alpha[NW][4];
+    // hold all heads in every lane (HPW = 8: heads 4 (g % 2) .. + 3).
+    __shared__ __attribute__((aligned(16))) float s_alpha[NW][kPHeads];
 
     const int t_begin = split * p.chunk;
     const int t_end = min(t_begin + p.chunk, p.seqlen);
@@ -579,7 +609,7 @@ void decode_attention_mfma_kernel(AttnParams p) {
     auto step = [&](const MfmaTile<F>& tile, const int t0) {
 
         // ---- scores for the tile's two 16-token blocks ----
-        float s[2];
+        float s[HPL][2];
         if constexpr (F == KvFormat::I4) {
             if (tile.grp != cur_group) {   // wave-uniform; the scales came with the tile
                 cur_group = tile.grp;
@@ -606,53 +636,68 @@ void decode_attention_mfma_kernel(AttnParams p) {
             const bool valid = (t0 + 16 * blk + c) < w1;
             float sc = p.scale_log2;
             if constexpr (F == KvFormat::I8) sc *= h2f(tile.ks[blk]);
-            const float dot = (F == KvFormat::I4) ? acc[0] + acc[1] : acc[0];
-            s[blk] = valid ? dot * sc : -INFINITY;
+            if constexpr (HPL == 2) {
+                s[0][blk] = valid ? ((F == KvFormat::I4) ? acc[0] + acc[1] : acc[0]) * sc : -INFINITY;
+                s[HPL - 1][blk] = valid ? ((F == KvFormat::I4) ? acc[2] + acc[3] : acc[1]) * sc : -INFINITY;
+            } else {
+                const float dot = (F == KvFormat::I4) ? acc[0] + acc[1] : acc[0];
+                s[0][blk] = valid ? dot * sc : -INFINITY;
+            }
         }
 
-        // ---- online softmax of lane group g's head over the 32 tokens ----
-        const float tmax = row16_max(fmaxf(s[0], s[1]));
-        const float mn = fmaxf(m_run, tmax);
-        const float msafe = (mn == -INFINITY) ? 0.0f : mn;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - msafe);
-        const bool rescale = __builtin_amdgcn_ballot_w64(mn != m_run) != 0;   // wave-uniform
-        m_run = mn;
-        const float pr0 = __builtin_amdgcn_exp2f(s[0] - msafe);
-        const float pr1 = __builtin_amdgcn_exp2f(s[1] - msafe);
-        l_run = fmaf(l_run, alpha, pr0 + pr1);
+        // ---- online softmax of lane group g's heads over the 32 tokens ----
+        float alpha[HPL], pr[HPL][2];
+        bool rescale = false;   // wave-uniform
+#pragma unroll
+        for (int i = 0; i < HPL; ++i) {
+            const float tmax = row16_max(fmaxf(s[i][0], s[i][1]));
+            const float mn = fmaxf(m_run[i], tmax);
+            const float msafe = (mn == -INFINITY) ? 0.0f : mn;
+            alpha[i] = __builtin_amdgcn_exp2f(m_run[i] - msafe);
+            rescale |= __builtin_amdgcn_ballot_w64(mn != m_run[i]) != 0;
+            m_run[i] = mn;
+            pr[i][0] = __builtin_amdgcn_exp2f(s[i][0] - msafe);
+            pr[i][1] = __builtin_amdgcn_exp2f(s[i][1] - msafe);
+            l_run[i] = fmaf(l_run[i], alpha[i], pr[i][0] + pr[i][1]);
+        }
 
-        // ---- p and alpha -> LDS (lane group g writes head g) -> A operand ----
+        // ---- p and alpha -> LDS (lane group g writes heads g, g + 4) -> A operand ----
         if (g < HPW) {
             float f0 = MfmaTile<F>::kPScale, f1 = MfmaTile<F>::kPScale;
             if constexpr (F != KvFormat::F16) {
                 f0 *= h2f(tile.vs[0]);
                 f1 *= h2f(tile.vs[1]);
             }
-            // x - fp16(x) is exact in fp32; rounding it to fp16 leaves a
-            // relative error of 2^-11 of a term that is itself <= 2^-11 x.
-            const float x0 = pr0 * f0, x1 = pr1 * f1;
-            const uint16_t h0 = f2h_bits(x0), h1 = f2h_bits(x1);
             // INT4: PV's k-slot 8 kq + e holds token 4 e + kq (each V load
             // instruction then reads four adjacent 64-byte rows, whole lines).
             const int sl0 = (F == KvFormat::I4) ? 8 * (c & 3) + (c >> 2) : c;
             const int sl1 = (F == KvFormat::I4) ? sl0 + 4 : 16 + c;
-            s_p[wave][0][g][sl0] = h0;
-            s_p[wave][0][g][sl1] = h1;
-            s_p[wave][1][g][sl0] = f2h_bits(x0 - h2f(h0));
-            s_p[wave][1][g][sl1] = f2h_bits(x1 - h2f(h1));
-            if (c == 0) s_alpha[wave][g] = alpha;
+#pragma unroll
+            for (int i = 0; i < HPL; ++i) {
+                // x - fp16(x) is exact in fp32; rounding it to fp16 leaves a
+                // relative error of 2^-11 of a term that is itself <= 2^-11 x.
+                const float x0 = pr[i][0] * f0, x1 = pr[i][1] * f1;
+                const uint16_t h0 = f2h_bits(x0), h1 = f2h_bits(x1);
+                s_p[wave][0][g + 4 * i][sl0] = h0;
+                s_p[wave][0][g + 4 * i][sl1] = h1;
+                s_p[wave][1][g + 4 * i][sl0] = f2h_bits(x0 - h2f(h0));
+                s_p[wave][1][g + 4 * i][sl1] = f2h_bits(x1 - h2f(h1));
+                if (c == 0) s_alpha[wave][g + 4 * i] = alpha[i];
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const f16x8 pa = as_f16x8(load16(&s_p[wave][kPlaneRows ? (c >> 2) & 1 : 0][c % HPW][8 * g]));
+        const int plane = kPlaneRows ? (HPL == 2 ? c >> 3 : (c >> 2) & 1) : 0;
+        const f16x8 pa = as_f16x8(load16(&s_p[wave][plane][c % HPW][8 * g]));
         const f16x8 pl = kPlaneRows ? pa : as_f16x8(load16(&s_p[wave][1][c % HPW][8 * g]));
         if (rescale) {
-            // PV row 4g + i is head i % HPW (PV's A row m = head m % HPW).
-            const f32x4 al = *reinterpret_cast<const f32x4*>(&s_alpha[wave][0]);
+            // PV row 4g + i is head i % HPW (PV's A row m = head m % HPW), or
+            // with HPW = 8 head 4 (g % 2) + i.
+            const f32x4 al = *reinterpret_cast<const f32x4*>(&s_alpha[wave][HPL == 2 ? 4 * (g & 1) : 0]);
             float a4[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a4[i] = al[i % HPW];
+            for (int i = 0; i < 4; ++i) a4[i] = al[HPL == 2 ? i : i % HPW];
 #pragma unroll
             for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -739,20 +784,25 @@ void decode_attention_mfma_kernel(AttnParams p) {
     }
 
     // ---- merge the wave states through LDS ----
-    const float l_tot = row16_sum(l_run);   // lane group g: head g's denominator
+    float l_tot[HPL];   // lane group g: the denominators of its heads
+#pragma unroll
+    for (int i = 0; i < HPL; ++i) l_tot[i] = row16_sum(l_run[i]);
 
     __shared__ __attribute__((aligned(16))) float s_o[NW][HPW][kHeadDim];
     __shared__ float s_m[NW][HPW];
     __shared__ float s_l[NW][HPW];
     __shared__ uint32_t s_last;
     constexpr float kInvP = 1.0f / MfmaTile<F>::kPScale;
-    if constexpr (kPlaneRows) {   // hi + lo planes: lane group g's PV rows plus lane group g ^ 1's
+    if constexpr (kPlaneRows) {   // hi + lo planes: lane group g's PV rows plus lane group g ^ 1's (HPW = 8: g ^ 2's)
+        constexpr int kOther = HPL == 2 ? 32 : 16;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[j][i] += __shfl_xor(o[j][i], 16);
+            for (int i = 0; i < 4; ++i) o[j][i] += __shfl_xor(o[j][i], kOther);
+        if constexpr (F != KvFormat::F16) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sum_p[i] += __shfl_xor(sum_p[i], 16);
+            for (int i = 0; i < 4; ++i) sum_p[i] += __shfl_xor(sum_p[i], kOther);
+        }
     }
     if constexpr (F != KvFormat::F16) {
 #pragma unroll
@@ -761,18 +811,21 @@ void decode_attention_mfma_kernel(AttnParams p) {
             for (int i = 0; i < 4; ++i)
                 o[j][i] = (o[j][i] - MfmaTile<F>::kVBias[j & 1] * sum_p[i]) * MfmaTile<F>::kVUnscale[j & 1];
     }
-    if (g == 0) {
+    if (g < HPL) {   // HPW = 8: lane group g holds heads 4g .. 4g + 3
 #pragma unroll
-        for (int i = 0; i < HPW; ++i)
+        for (int i = 0; i < HPW / HPL; ++i)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s_o[wave][i][8 * c + j] = o[j][i] * kInvP;
+            for (int j = 0; j < 8; ++j) s_o[wave][4 * g + i][8 * c + j] = o[j][i] * kInvP;
     }
     if (c == 0 && g < HPW) {
-        s_m[wave][g] = m_run;
-        s_l[wave][g] = l_tot;
+#pragma unroll
+        for (int i = 0; i < HPL; ++i) {
+            s_m[wave][g + 4 * i] = m_run[i];
+            s_l[wave][g + 4 * i] = l_tot[i];
+        }
     }
     __syncthreads();
-    finish_split<NW, HPW, NW * kWave>(p, s_o, s_m, s_l, &s_last, b, kvh, hchunk, split, head0);
+    finish_split<NW, HPW, NW * kWave, PAD>(p, s_o, s_m, s_l, &s_last, b, kvh, hchunk, split, head0);
 }
 
 // ===========================================================================
@@ -822,7 +875,7 @@ struct F16HalfTile {
     }
 };
 
-template <int HPW, int NW>
+template <int HPW, int NW, bool PAD>
 __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_attention_f16h_kernel(AttnParams p) {
     const int split = blockIdx.x;
@@ -834,17 +887,27 @@ void decode_attention_f16h_kernel(AttnParams p) {
     const int lane = tid & 63;
     const int g = lane >> 4;
     const int c = lane & 15;
-    const int head0 = kvh * p.gqa + hchunk * HPW;
-    const uint16_t* qrow = p.q + ((long)b * p.n_heads + head0 + ((c >> 2) % HPW)) * kHeadDim;
+    // Heads and rows as in the 32-token kernel.
+    constexpr int HPL = HPW > 4 ? 2 : 1;
+    const int head0 = chunk_head0<HPW, PAD>(p, kvh, hchunk);
+    const int nh = chunk_heads<HPW, PAD>(p, hchunk);
+    const int hrow = HPL == 2 ? (c >> 2) + 4 * (c & 1) : (c >> 2) % HPW;
+    const uint16_t* qrow = p.q + ((long)b * p.n_heads + head0 + (PAD ? min(hrow, nh - 1) : hrow)) * kHeadDim;
     f16x8 qa[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) qa[ks] = as_f16x8(load16(qrow + 32 * ks + 8 * g));
     f32x4 o[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) o[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = -INFINITY, l_run = 0.0f;
-    __shared__ __attribute__((aligned(16))) uint16_t s_p[NW][2][4][kHalfTile];
-    __shared__ __attribute__((aligned(16))) float s_alpha[NW][4];
+    float m_run[HPL], l_run[HPL];
+#pragma unroll
+    for (int i = 0; i < HPL; ++i) {
+        m_run[i] = -INFINITY;
+        l_run[i] = 0.0f;
+    }
+    constexpr int kPHeads = HPL == 2 ? 8 : 4;
+    __shared__ __attribute__((aligned(16))) uint16_t s_p[NW][2][kPHeads][kHalfTile];
+    __shared__ __attribute__((aligned(16))) float s_alpha[NW][kPHeads];
 
     const int w0 = (split + p.n_splits * wave) * kHalfTile;
     const int w1 = p.seqlen;
@@ -865,33 +928,45 @@ void decode_attention_f16h_kernel(AttnParams p) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) acc = mfma16x16x32(qa[ks], as_f16x8(tile.k[ks]), acc);
-        const float s = (t0 + c) < w1 ? acc[0] * p.scale_log2 : -INFINITY;
-        const float tmax = row16_max(s);
-        const float mn = fmaxf(m_run, tmax);
-        const float msafe = (mn == -INFINITY) ? 0.0f : mn;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - msafe);
-        const bool rescale = __builtin_amdgcn_ballot_w64(mn != m_run) != 0;
-        m_run = mn;
-        const float pr = __builtin_amdgcn_exp2f(s - msafe);
-        l_run = fmaf(l_run, alpha, pr);
+        float alpha[HPL], pr[HPL];
+        bool rescale = false;   // wave-uniform
+#pragma unroll
+        for (int i = 0; i < HPL; ++i) {
+            const float s = (t0 + c) < w1 ? acc[i] * p.scale_log2 : -INFINITY;
+            const float tmax = row16_max(s);
+            const float mn = fmaxf(m_run[i], tmax);
+            const float msafe = (mn == -INFINITY) ? 0.0f : mn;
+            alpha[i] = __builtin_amdgcn_exp2f(m_run[i] - msafe);
+            rescale |= __builtin_amdgcn_ballot_w64(mn != m_run[i]) != 0;
+            m_run[i] = mn;
+            pr[i] = __builtin_amdgcn_exp2f(s - msafe);
+            l_run[i] = fmaf(l_run[i], alpha[i], pr[i]);
+        }
         if (g < HPW) {
-            const float xv = pr * MfmaTile<KvFormat::F16>::kPScale;
-            const uint16_t h = f2h_bits(xv);
-            s_p[wave][0][g][c] = h;
-            s_p[wave][1][g][c] = f2h_bits(xv - h2f(h));
-            if (c == 0) s_alpha[wave][g] = alpha;
+#pragma unroll
+            for (int i = 0; i < HPL; ++i) {
+                const float xv = pr[i] * MfmaTile<KvFormat::F16>::kPScale;
+                const uint16_t h = f2h_bits(xv);
+                s_p[wave][0][g + 4 * i][c] = h;
+                s_p[wave][1][g + 4 * i][c] = f2h_bits(xv - h2f(h));
+                if (c == 0) s_alpha[wave][g + 4 * i] = alpha[i];
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // A operand of PV: row c (head c % HPW), tokens 4 g .. 4 g + 3.
-        const f16x4 pa = __builtin_bit_cast(f16x4, *reinterpret_cast<const u32x2*>(&s_p[wave][0][c % HPW][4 * g]));
-        const f16x4 pl = __builtin_bit_cast(f16x4, *reinterpret_cast<const u32x2*>(&s_p[wave][1][c % HPW][4 * g]));
+        // A operand of PV: row c (head c % HPW; HPW = 8: plane c / 8 of it),
+        // tokens 4 g .. 4 g + 3.
+        const f16x4 pa = __builtin_bit_cast(
+            f16x4, *reinterpret_cast<const u32x2*>(&s_p[wave][HPL == 2 ? c >> 3 : 0][c % HPW][4 * g]));
+        f16x4 pl = pa;
+        if constexpr (HPL == 1)
+            pl = __builtin_bit_cast(f16x4, *reinterpret_cast<const u32x2*>(&s_p[wave][1][c % HPW][4 * g]));
         if (rescale) {
-            const f32x4 al = *reinterpret_cast<const f32x4*>(&s_alpha[wave][0]);
+            const f32x4 al = *reinterpret_cast<const f32x4*>(&s_alpha[wave][HPL == 2 ? 4 * (g & 1) : 0]);
             float a4[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a4[i] = al[i % HPW];
+            for (int i = 0; i < 4; ++i) a4[i] = al[HPL == 2 ? i : i % HPW];
 #pragma unroll
             for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -903,7 +978,7 @@ void decode_attention_f16h_kernel(AttnParams p) {
         for (int j = 0; j < 8; ++j) {
             const f16x4 vb = tile.vop(j);
             o[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa, vb, o[j], 0, 0, 0);
-            o[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, vb, o[j], 0, 0, 0);
+            if constexpr (HPL == 1) o[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, vb, o[j], 0, 0, 0);
         }
     };
 
@@ -927,24 +1002,35 @@ void decode_attention_f16h_kernel(AttnParams p) {
         }
     }
 
-    const float l_tot = row16_sum(l_run);
+    float l_tot[HPL];
+#pragma unroll
+    for (int i = 0; i < HPL; ++i) l_tot[i] = row16_sum(l_run[i]);
+    if constexpr (HPL == 2) {   // hi + lo planes
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[j][i] += __shfl_xor(o[j][i], 32);
+    }
     __shared__ __attribute__((aligned(16))) float s_o[NW][HPW][kHeadDim];
     __shared__ float s_m[NW][HPW];
     __shared__ float s_l[NW][HPW];
     __shared__ uint32_t s_last;
     constexpr float kInvP = 1.0f / MfmaTile<KvFormat::F16>::kPScale;
-    if (g == 0) {
+    if (g < HPL) {
 #pragma unroll
-        for (int i = 0; i < HPW; ++i)
+        for (int i = 0; i < HPW / HPL; ++i)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s_o[wave][i][8 * c + j] = o[j][i] * kInvP;
+            for (int j = 0; j < 8; ++j) s_o[wave][4 * g + i][8 * c + j] = o[j][i] * kInvP;
     }
     if (c == 0 && g < HPW) {
-        s_m[wave][g] = m_run;
-        s_l[wave][g] = l_tot;
+#pragma unroll
+        for (int i = 0; i < HPL; ++i) {
+            s_m[wave][g + 4 * i] = m_run[i];
+            s_l[wave][g + 4 * i] = l_tot[i];
+        }
     }
     __syncthreads();
-    finish_split<NW, HPW, NW * kWave>(p, s_o, s_m, s_l, &s_last, b, kvh, hchunk, split, head0);
+    finish_split<NW, HPW, NW * kWave, PAD>(p, s_o, s_m, s_l, &s_last, b, kvh, hchunk, split, head0);
 }
 
 // ===========================================================================
@@ -1133,7 +1219,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_valu_kernel(Att
         }
     }
     __syncthreads();
-    finish_split<kRows, HPW, kAttnThreads>(p, s_o, s_m, s_l, &s_last, b, kvh, hchunk, split, head0);
+    finish_split<kRows, HPW, kAttnThreads, false>(p, s_o, s_m, s_l, &s_last, b, kvh, hchunk, split, head0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1142,21 +1228,47 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_valu_kernel(Att
 
 namespace {
 
-int heads_per_wg(int gqa) {
-    if (gqa % 4 == 0) return 4;
-    if (gqa % 2 == 0) return 2;
-    return 1;
+// Heads per workgroup. MFMA kernels: all query heads of a kv head together up
+// to `most` (4 or 8) of them, more in equal chunks; the 16 rows of a matrix
+// operand cost the same for 3 heads as for 4 and for 5 as for 8. VALU kernel,
+// whose work grows with every head: the power of two up to 4 that divides.
+void head_chunks(int gqa, bool mfma, int most, AttnPlan& pl) {
+    if (mfma) {
+        pl.n_hchunks = (gqa + most - 1) / most;
+        pl.heads_per_chunk = (gqa + pl.n_hchunks - 1) / pl.n_hchunks;
+        pl.hpw = pl.heads_per_chunk > 4 ? 8 : pl.heads_per_chunk > 2 ? 4 : pl.heads_per_chunk;
+        return;
+    }
+    pl.hpw = gqa % 4 == 0 ? 4 : gqa % 2 == 0 ? 2 : 1;
+    pl.heads_per_chunk = pl.hpw;
+    pl.n_hchunks = gqa / pl.hpw;
 }
 
 }  // namespace
 
-AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen) {
+// (split, slot group) pairs of 8 heads that fit LLMIK_NOALLOC_SCRATCH_BYTES:
+// per head 128 fp32 outputs and (m, l), after the counters and two alignments.
+constexpr long kMaxWideSlots =
+    (long)((LLMIK_NOALLOC_SCRATCH_BYTES - kCounterBytes - 512) / (8 * (kHeadDim + 2) * sizeof(float)));
+
+AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, bool mfma) {
     AttnPlan pl{};
     const int gqa = n_heads / n_kv_heads;
-    pl.hpw = heads_per_wg(gqa);
-    pl.n_hchunks = gqa / pl.hpw;
-    const long base_wgs = (long)batch * n_kv_heads * pl.n_hchunks;
     const int cus = device_cu_count();
+    const long target = (long)kAttnWgsPerCu * cus;
+    const long splits8 = ((long)seqlen + 8 * kTile - 1) / (8 * kTile);
+    // One workgroup for up to 8 heads of a kv head reads its cache once; with
+    // chunks of 4, 2 or 1 heads (the largest that divides the head count, the
+    // rule before) every chunk read it again, through L2 at best. us, fp16:
+    // H=64 Hkv=8 (4 + 4) B=12 S=3001 49.4 -> 35.7, B=32 S=2048 78.1 -> 40.1;
+    // H=28 Hkv=4 (7 x 1) B=16 S=2000 64.0 -> 14.9; H=40 Hkv=8 (5 x 1) B=8
+    // S=4096 118 -> 27.2; H=24 Hkv=8 (3 x 1) B=20 S=1500 51.9 -> 26.7. INT8
+    // H=64 B=8 S=4096 23.8 -> 15.2, INT4 g128 B=32 S=4096 50.8 -> 32.3. If
+    // even one step per wave would leave CUs idle, chunks of up to 4 heads
+    // (twice the workgroups) finish sooner: INT4 H=64 B=2 S=2048 8.95 against
+    // 8.35, INT8 B=1 S=2000 7.6 against 7.5.
+    head_chunks(gqa, mfma, (long)batch * n_kv_heads * ((gqa + 7) / 8) * splits8 < target ? 4 : 8, pl);
+    const long base_wgs = (long)batch * n_kv_heads * pl.n_hchunks;
     // Aim for kAttnWgsPerCu workgroups per CU. Calls that must split the
     // sequence to fill the chip use 8-wave workgroups (more loads in flight
     // per CU); otherwise 4 waves. Every split
@@ -1166,8 +1278,6 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen) {
     // the combine to at most 8 partials: at B=1, S=1024 the 8 splits took
     // 6.9 us against 9.0 us for 4; at B=1, S=4096 32 splits took 12.6 us
     // against 10.4 us for 16 (the combine grows with the split count).
-    const long target = (long)kAttnWgsPerCu * cus;
-    const long splits8 = ((long)seqlen + 8 * kTile - 1) / (8 * kTile);
     const bool short_seq = base_wgs * splits8 < target && 2 * splits8 <= 8;
     pl.waves = (base_wgs < target && !short_seq) ? 8 : 4;
     // Splits that would give each of 8 waves a single 32-token tile run as
@@ -1183,6 +1293,9 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen) {
     if (want > max_useful) want = max_useful;
     if (want > kMaxAttnSplits) want = kMaxAttnSplits;
     if (base_wgs > kMaxCounters) want = 1;   // enough workgroups without splitting
+    // Partials of 8 heads per workgroup stay within the workspace that 4 took
+    // (and within the static scratch of the entry point without a workspace).
+    if (pl.hpw == 8) want = std::min(want, kMaxWideSlots / base_wgs);
     if (want < 1) want = 1;
     int chunk = (int)((seqlen + want - 1) / want);
     chunk = ((chunk + step - 1) / step) * step;
@@ -1217,7 +1330,10 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen) {
 // two 32-token tiles per wave unless the workgroups have 4 waves. It takes
 // the faster form at 24 of these 26 shapes (the earlier rule, 2-8 tiles per
 // wave, at 16). The override (llmik_attention_set_plan_override) forces
-// either.
+// either. Chunks of 3 heads keep 32-token tiles (B=8 Hkv=8, 32 -> 16: S=2000
+// 13.9 -> 14.0, S=4096 23.6 -> 28.0); with 8 heads per workgroup one tile per
+// wave is even (H=64, B=4 S=2000: 10.26 -> 10.31) and H=64, B=32 S=2048 gains
+// (42.8 -> 40.2).
 namespace {
 std::atomic<int> g_f16_tiles{-1};   // -1: the rule, 0: 32-token tiles, 1: 16-token tiles
 }  // namespace
@@ -1232,33 +1348,56 @@ static bool use_f16_half_tiles(const AttnPlan& pl, int seqlen) {
     const long tiles = (seqlen + kTile - 1) / kTile;
     const long per_wave = (tiles + (long)pl.n_splits * pl.waves - 1) / ((long)pl.n_splits * pl.waves);
     const long wgs = (long)pl.n_slot_groups * pl.n_splits;
-    return pl.n_slot_groups >= 32 && wgs % device_cu_count() == 0 && (per_wave >= 2 || pl.waves == 4);
+    if (pl.heads_per_chunk == 3) return false;
+    return pl.n_slot_groups >= 32 && wgs % device_cu_count() == 0 &&
+           (per_wave >= 2 || pl.waves == 4 || pl.hpw == 8);
 }
 
-template <KvFormat F, int HPW>
-static void launch_kernel(const AttnParams& p, dim3 grid, bool mfma, int waves, bool half, hipStream_t stream) {
-    if (F == KvFormat::F16 && mfma && half) {
-        if (waves == 8)
-            hipLaunchKernelGGL((decode_attention_f16h_kernel<HPW, 8>), grid, dim3(8 * kWave), 0, stream, p);
-        else
-            hipLaunchKernelGGL((decode_attention_f16h_kernel<HPW, 4>), grid, dim3(4 * kWave), 0, stream, p);
+template <KvFormat F, int HPW, bool PAD>
+static void launch_mfma(const AttnParams& p, dim3 grid, int waves, bool half, hipStream_t stream) {
+    if constexpr (F == KvFormat::F16) {
+        if (half) {
+            if (waves == 8)
+                hipLaunchKernelGGL((decode_attention_f16h_kernel<HPW, 8, PAD>), grid, dim3(8 * kWave), 0, stream, p);
+            else
+                hipLaunchKernelGGL((decode_attention_f16h_kernel<HPW, 4, PAD>), grid, dim3(4 * kWave), 0, stream, p);
+            return;
+        }
+    }
+    if (waves == 8)
+        hipLaunchKernelGGL((decode_attention_mfma_kernel<F, HPW, 8, PAD>), grid, dim3(8 * kWave), 0, stream, p);
+    else
+        hipLaunchKernelGGL((decode_attention_mfma_kernel<F, HPW, 4, PAD>), grid, dim3(4 * kWave), 0, stream, p);
+}
+
+template <KvFormat F>
+static void launch_kernel(const AttnParams& p, const AttnPlan& pl, dim3 grid, bool mfma, bool half,
+                          hipStream_t stream) {
+    if (!mfma) {
+        const dim3 block(kAttnThreads);
+        if (pl.hpw == 4) hipLaunchKernelGGL((decode_attention_valu_kernel<F, 4>), grid, block, 0, stream, p);
+        else if (pl.hpw == 2) hipLaunchKernelGGL((decode_attention_valu_kernel<F, 2>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((decode_attention_valu_kernel<F, 1>), grid, block, 0, stream, p);
         return;
     }
-    if (mfma && waves == 8) {
-        hipLaunchKernelGGL((decode_attention_mfma_kernel<F, HPW, 8>), grid, dim3(8 * kWave), 0,
-                           stream, p);
-    } else if (mfma) {
-        hipLaunchKernelGGL((decode_attention_mfma_kernel<F, HPW, 4>), grid, dim3(4 * kWave), 0,
-                           stream, p);
-    } else {
-        hipLaunchKernelGGL((decode_attention_valu_kernel<F, HPW>), grid, dim3(kAttnThreads), 0,
-                           stream, p);
-    }
+    const bool pad = pl.heads_per_chunk * pl.n_hchunks != p.gqa || pl.heads_per_chunk != pl.hpw;
+    if (pl.hpw == 8 && pad) launch_mfma<F, 8, true>(p, grid, pl.waves, half, stream);
+    else if (pl.hpw == 8) launch_mfma<F, 8, false>(p, grid, pl.waves, half, stream);
+    else if (pl.hpw == 4 && pad) launch_mfma<F, 4, true>(p, grid, pl.waves, half, stream);
+    else if (pl.hpw == 4) launch_mfma<F, 4, false>(p, grid, pl.waves, half, stream);
+    else if (pl.hpw == 2) launch_mfma<F, 2, false>(p, grid, pl.waves, half, stream);
+    else launch_mfma<F, 1, false>(p, grid, pl.waves, half, stream);
 }
 
 template <KvFormat F>
 static int launch_attention(const AttnLaunch& a, hipStream_t stream) {
-    const AttnPlan pl = plan_attention(a.batch, a.n_heads, a.n_kv_heads, a.seqlen);
+    // The MFMA path keeps each 32-token tile inside one INT4 K-scale group,
+    // and addresses a (batch, kv head) slab with 32-bit buffer offsets.
+    const int group_size = a.group_size > 0 ? a.group_size : 1;
+    const long row_bytes = (F == KvFormat::F16) ? 2 * kHeadDim : (F == KvFormat::I8 ? kHeadDim : kHeadDim / 2);
+    const bool mfma = ((F != KvFormat::I4) || (group_size % kTile == 0)) &&
+                      (long)a.kv_buf_len * row_bytes < (1L << 32);
+    const AttnPlan pl = plan_attention(a.batch, a.n_heads, a.n_kv_heads, a.seqlen, mfma);
     if (pl.n_splits > 1 && a.workspace_bytes < pl.workspace_bytes) {
         return set_error(LLMIK_ERR_WORKSPACE, "workspace too small for this attention call");
     }
@@ -1277,26 +1416,18 @@ static int launch_attention(const AttnLaunch& a, hipStream_t stream) {
     p.n_kv_heads = a.n_kv_heads;
     p.seqlen = a.seqlen;
     p.kv_buf_len = a.kv_buf_len;
-    p.group_size = a.group_size > 0 ? a.group_size : 1;
+    p.group_size = group_size;
     p.n_groups = a.n_groups;
     p.n_splits = pl.n_splits;
     p.chunk = pl.chunk;
     p.n_hchunks = pl.n_hchunks;
+    p.heads_per_chunk = pl.heads_per_chunk;
     p.gqa = a.n_heads / a.n_kv_heads;
     p.scale_log2 = a.softmax_scale * kLog2e;
 
-    // The MFMA path keeps each 32-token tile inside one INT4 K-scale group,
-    // and addresses a (batch, kv head) slab with 32-bit buffer offsets.
-    const long row_bytes = (F == KvFormat::F16) ? 2 * kHeadDim : (F == KvFormat::I8 ? kHeadDim : kHeadDim / 2);
-    const bool mfma = ((F != KvFormat::I4) || (p.group_size % kTile == 0)) &&
-                      (long)a.kv_buf_len * row_bytes < (1L << 32);
     const bool half = (F == KvFormat::F16) && mfma && use_f16_half_tiles(pl, a.seqlen);
     dim3 grid(pl.n_splits, a.n_kv_heads * pl.n_hchunks, a.batch);
-    switch (pl.hpw) {
-        case 4: launch_kernel<F, 4>(p, grid, mfma, pl.waves, half, stream); break;
-        case 2: launch_kernel<F, 2>(p, grid, mfma, pl.waves, half, stream); break;
-        default: launch_kernel<F, 1>(p, grid, mfma, pl.waves, half, stream); break;
-    }
+    launch_kernel<F>(p, pl, grid, mfma, half, stream);
     return check_launch();
 }
 

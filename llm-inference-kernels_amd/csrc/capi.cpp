@@ -94,7 +94,11 @@ LLMIK_API size_t llmik_attention_workspace_size(int batch, int n_heads, int n_kv
     if (batch <= 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim != 128 ||
         n_heads % n_kv_heads != 0 || seqlen <= 0)
         return 0;
-    return plan_attention(batch, n_heads, n_kv_heads, seqlen).workspace_bytes;
+    // The size does not name the cache format: enough for the matrix-core
+    // kernels' plan and for the VALU kernel's.
+    const size_t mfma = plan_attention(batch, n_heads, n_kv_heads, seqlen, true).workspace_bytes;
+    const size_t valu = plan_attention(batch, n_heads, n_kv_heads, seqlen, false).workspace_bytes;
+    return mfma > valu ? mfma : valu;
 }
 
 LLMIK_API llmik_status llmik_decode_attention_f16(const void* q, const void* k, const void* v,

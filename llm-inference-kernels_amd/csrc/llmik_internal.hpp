@@ -28,8 +28,9 @@ int device_cu_count();
 
 // ---- attention -------------------------------------------------------------
 struct AttnPlan {
-    int hpw;             // query heads per workgroup
+    int hpw;             // query heads a workgroup computes (1, 2, 4 or 8)
     int n_hchunks;       // head chunks per kv head
+    int heads_per_chunk; // query heads of a chunk (<= hpw; the last chunk may hold fewer)
     int n_splits;        // KV splits per (batch, kv head, head chunk)
     int chunk;           // tokens per split (multiple of 32 * waves)
     int waves;           // waves per MFMA workgroup (4 or 8)
@@ -38,7 +39,8 @@ struct AttnPlan {
     size_t off_ml, off_o;
 };
 
-AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen);
+// mfma: the plan of the matrix-core kernels, else of the VALU kernel.
+AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, bool mfma);
 // fp16 tile size knob (see llmik_attention_set_plan_override).
 void set_attention_plan_override(int f16_half_tiles);
 // W4A16 plan knobs (see llmik_w4a16_set_plan_override).
