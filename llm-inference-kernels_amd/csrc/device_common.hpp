@@ -253,18 +253,72 @@ __device__ __forceinline__ float sym_scale(uint32_t absmax_bits, float qmax) {
     return s < 1.0e-8f ? 1.0e-8f : s;
 }
 
-// clamp(round(x / s), -qmax, qmax) as an integer code (r = 1 / s). A NaN
-// quotient (a NaN scale, or inf / inf) gives code 0, which is what torch's
-// float -> int8 conversion of NaN stores on x86; finite / inf is 0 already.
-// v_cvt_i32_f32 converts NaN to 0 and saturates out-of-range values (CDNA
-// ISA), so the conversion comes first and the clamp is one integer med3; it
-// is written as inline asm because a C++ float -> int conversion of NaN is
-// undefined behaviour the compiler may exploit.
-__device__ __forceinline__ int sym_code(float x, float s, float r, int qmax) {
-    const float v = quant_round(x, s, r);
-    int c;
-    asm("v_cvt_i32_f32 %0, %1" : "=v"(c) : "v"(v));
-    return min(max(c, -qmax), qmax);
+// ---- codes of fp16 values within the scale's range -----------------------------
+// The KV writers' form of quant_round: every |x| is at most the absmax that
+// gave s = max(absmax / QMAX, 1e-8), so |x / s| <= QMAX (1 + 2^-24) and no
+// clamp is needed. z = fma(x, r, 0) is the exact product x * r: with r within
+// 1 ulp of 1 / s (2^-23 relative) and the correctly rounded quotient within
+// 2^-24 of x / s, z is within QMAX * 1.5 * 2^-23 (1 + 2^-23) of that quotient:
+// below 2^-19 for QMAX = 7 and 2^-15 for 127. So rint(z) is the code unless z
+// lies that close to a half-integer; within twice that (kTieWindow, which
+// also covers the rounding of d) the true division decides.
+// fma(x, r, kCodeMagic) rounds z to an integer, half to even, in the low bits
+// of an fp32 word (1.5 * 2^23: two's complement there), converting x from
+// fp16, multiplying and rounding in one instruction; d = fma(x, r, -code) is
+// the distance that the tie test needs. About 5 instructions a value with the
+// packing, against 12 with a product, rint, a tie test, a conversion and a
+// clamp each. The tie test branches once for N values and then per value.
+// NaN: an fp16 NaN has no payload below bit 13 of its fp32 form and neither has
+// the default NaN of 0 * inf, so the code bits of a NaN word are 0, which is
+// what torch's float -> int8 conversion of NaN stores on x86; finite / inf
+// gives z = 0, code 0; comparisons with NaN send nothing to the division.
+constexpr float kCodeMagic = 12582912.0f;
+template <int QMAX>
+constexpr float kTieWindow = QMAX == 7 ? 0x1p-18f : 0x1p-14f;
+
+// Code words of the 2 N fp16 values in w[N]: value e has scale s[e % NS] and
+// reciprocal r[e % NS]; the code is the low byte / nibble of t[e].
+template <int QMAX, int N, int NS>
+__device__ __forceinline__ void code_words(const uint32_t (&w)[N], const float (&s)[NS], const float (&r)[NS],
+                                           uint32_t (&t)[2 * N]) {
+    static_assert(QMAX == 7 || QMAX == 127, "kTieWindow is derived for these");
+    constexpr float kNear = 0.5f - kTieWindow<QMAX>;
+    float d[2 * N], worst = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 2 * N; ++e) {
+        const float x = (float)as_f16x2(w[e >> 1])[e & 1];
+        const float v = fmaf(x, r[e % NS], kCodeMagic);
+        d[e] = fabsf(fmaf(x, r[e % NS], -(v - kCodeMagic)));
+        worst = fmaxf(worst, d[e]);
+        t[e] = __float_as_uint(v);
+    }
+    if (worst >= kNear) {
+#pragma unroll
+        for (int e = 0; e < 2 * N; ++e) {
+            const float x = (float)as_f16x2(w[e >> 1])[e & 1];
+            if (d[e] >= kNear) t[e] = __float_as_uint(__builtin_rintf(x / s[e % NS]) + kCodeMagic);
+        }
+    }
+}
+
+// Eight code words -> one dword of nibbles (element e in bits 4e .. 4e + 3).
+__device__ __forceinline__ uint32_t pack_nibbles(const uint32_t* t) {
+    uint32_t b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = (t[2 * i] & 0xFu) | (t[2 * i + 1] << 4);   // low byte
+    return perm_b32(perm_b32(b[3], b[2], 0x0C0C0400u), perm_b32(b[1], b[0], 0x0C0C0400u), 0x05040100u);
+}
+
+// Four code words -> one dword of bytes.
+__device__ __forceinline__ uint32_t pack_bytes(const uint32_t* t) {
+    return perm_b32(perm_b32(t[3], t[2], 0x0C0C0400u), perm_b32(t[1], t[0], 0x0C0C0400u), 0x05040100u);
+}
+
+// max(m, |x|) of packed fp16 pairs as bit patterns: with the sign cleared, the
+// unsigned order is the order of the magnitudes, NaN above +inf.
+__device__ __forceinline__ uint32_t max_abs2(uint32_t m, uint32_t x) {
+    const u16x2 a = __builtin_bit_cast(u16x2, m), b = __builtin_bit_cast(u16x2, x & 0x7FFF7FFFu);
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(a, b));
 }
 
 }  // namespace llmik

@@ -60,7 +60,9 @@ struct TokenMap {
 // tokens per lane group), same bits, on one box (us): INT8 B=8 S=4096 18.87
 // -> 18.50, INT4 V 17.79 -> 16.25, INT8 / INT4 V B=64 131.8 / 120.7 ->
 // 125.5 / 110.2, S=1000 6.62 / 6.48 -> 6.27 / 5.95; two tokens per group
-// (64 per workgroup) was slower for INT8 (20.4) and at small shapes.
+// (64 per workgroup) was slower for INT8 (20.4) and at small shapes. With
+// code_words: INT8 / INT4 V B=8 S=4096 18.1 / 15.4 -> 17.6 / 14.8, INT4 V
+// B=64 108.8 -> 104.2, INT8 B=64 125.2 -> 125.8 (bound by the stream).
 constexpr int kTokensPerRow8 = 1;
 
 __device__ __forceinline__ uint32_t row8_umax(uint32_t v) {
@@ -92,56 +94,81 @@ __global__ __launch_bounds__(kWriterThreads) void quantize_per_token_kernel(
     for (int i = 0; i < kTokensPerRow8; ++i) {
         const long flat = blk + kGroups * i + grp;
         // |x| of the 16 fp16 values as bit patterns, packed max per half.
-        uint32_t m = 0u;
+        uint32_t w[8], m = 0u;
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const uint32_t a = raw[i][h][d] & 0x7FFF7FFFu;
-                m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(
-                        __builtin_bit_cast(u16x2, m), __builtin_bit_cast(u16x2, a)));
-            }
+        for (int d = 0; d < 8; ++d) {
+            w[d] = raw[i][d >> 2][d & 3];
+            m = max_abs2(m, w[d]);
+        }
         const uint32_t m16 = max(m & 0xFFFFu, m >> 16);
         const uint32_t amax16 = row8_umax(m16);
         const float amax = h2f((uint16_t)amax16);   // exact; NaN stays NaN, inf stays inf
         const float sc = sym_scale(__float_as_uint(amax), (float)QMAX);
-        const float rcp = recip_approx(sc);
-        float xf[16];
-        f16x8_to_f32(raw[i][0], xf);
-        f16x8_to_f32(raw[i][1], xf + 8);
-        int code[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) code[e] = sym_code(xf[e], sc, rcp, QMAX);
+        const float s1[1] = {sc}, r1[1] = {recip_approx(sc)};
+        uint32_t code[16];
+        code_words<QMAX>(w, s1, r1, code);
         if (flat < rows) {
             const long row = MAPPED ? map.dst((uint32_t)flat) : flat;
             if constexpr (PACK4) {
-                uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    w0 |= (uint32_t)(code[e] & 0xF) << (4 * e);
-                    w1 |= (uint32_t)(code[8 + e] & 0xF) << (4 * e);
-                }
-                __builtin_nontemporal_store(w0, reinterpret_cast<uint32_t*>(q + row * 64 + 4 * c));
-                __builtin_nontemporal_store(w1, reinterpret_cast<uint32_t*>(q + row * 64 + 32 + 4 * c));
+                __builtin_nontemporal_store(pack_nibbles(code), reinterpret_cast<uint32_t*>(q + row * 64 + 4 * c));
+                __builtin_nontemporal_store(pack_nibbles(code + 8), reinterpret_cast<uint32_t*>(q + row * 64 + 32 + 4 * c));
             } else {
-                uint32_t w[4];
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-                    w[d] = (uint32_t)(code[4 * d] & 0xFF) | ((uint32_t)(code[4 * d + 1] & 0xFF) << 8) |
-                           ((uint32_t)(code[4 * d + 2] & 0xFF) << 16) | ((uint32_t)(code[4 * d + 3] & 0xFF) << 24);
-                __builtin_nontemporal_store(u32x2{w[0], w[1]}, reinterpret_cast<u32x2*>(q + row * 128 + 8 * c));
-                __builtin_nontemporal_store(u32x2{w[2], w[3]}, reinterpret_cast<u32x2*>(q + row * 128 + 64 + 8 * c));
+                __builtin_nontemporal_store(u32x2{pack_bytes(code), pack_bytes(code + 4)},
+                                            reinterpret_cast<u32x2*>(q + row * 128 + 8 * c));
+                __builtin_nontemporal_store(u32x2{pack_bytes(code + 8), pack_bytes(code + 12)},
+                                            reinterpret_cast<u32x2*>(q + row * 128 + 64 + 8 * c));
             }
             if (c == 0) scale[row] = f2h_bits(sc);
         }
     }
 }
 
-// K per channel, group-wise: one workgroup per (batch, kv_head, group). 16
-// rows of 16 lanes: row r holds the group's tokens r, r+16, ... (at most
-// TPR of them, group_size <= 16 * TPR) in registers; lane c owns channels
-// 8c..8c+7. The per-channel absmax is merged across rows in LDS, then the
-// codes are formed from the registers: the input is read once.
+// The K writers' workgroup: 16 rows of 16 lanes, lane c of a row owning
+// channels 8c..8c+7. Merges the rows' packed absmax (fp16 bit patterns, m) in
+// LDS, computes the 128 channels' scales and their reciprocals once, stores
+// the fp16 scales and hands each lane its channels'.
+struct KScales {
+    uint16_t maxes[16][128];
+    float scale[128], rcp[128];
+};
+__device__ __forceinline__ void k_group_scales(KScales& l, const uint32_t (&m)[4], uint16_t* __restrict__ scale,
+                                               float (&sv)[8], float (&rv)[8]) {
+    const int row = threadIdx.x >> 4;
+    const int c = threadIdx.x & 15;
+    *reinterpret_cast<u32x4*>(&l.maxes[row][8 * c]) = u32x4{m[0], m[1], m[2], m[3]};
+    __syncthreads();
+    if (threadIdx.x < 128) {
+        uint32_t a = 0u;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) a = max(a, (uint32_t)l.maxes[r][threadIdx.x]);
+        const float sc = sym_scale(__float_as_uint(h2f((uint16_t)a)), 7.0f);
+        l.scale[threadIdx.x] = sc;
+        l.rcp[threadIdx.x] = recip_approx(sc);
+        scale[threadIdx.x] = f2h_bits(sc);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        sv[e] = l.scale[8 * c + e];
+        rv[e] = l.rcp[8 * c + e];
+    }
+}
+
+// Dynamic LDS that, beside the static part, admits four workgroups to a CU's 160 KiB.
+constexpr size_t kWideGroupLds = 36 * 1024 - sizeof(KScales);
+static_assert(5 * (kWideGroupLds + sizeof(KScales)) > 160 * 1024 && 4 * (kWideGroupLds + sizeof(KScales)) <= 160 * 1024,
+              "four workgroups, not five");
+
+// K per channel, group-wise: one workgroup per (batch, kv_head, group). Row r
+// holds the group's tokens r, r+16, ... (at most TPR of them, group_size <=
+// 16 * TPR) in registers; the codes are formed from the registers: the input
+// is read once. Bound by the read + write stream. With code_words, packed
+// maxima and one reciprocal per channel (us, before -> now): B=8 Hkv=8 S=4096
+// g128 17.5 -> 16.7, g64 16.1 -> 15.5, g32 17.0 -> 15.7; B=64 g32 116 -> 109.
+// Groups of 65-128 tokens are held to 4 workgroups per CU by unused dynamic
+// LDS (kWideGroupLds; the registers would admit 6): B=64 108 -> 105, against
+// 113 with 6, 112 with 5 and 108.8 with 3, as more loads in flight only lengthen the
+// memory queues; B=8 is 2 % slower for it.
 template <int TPR>
 __global__ __launch_bounds__(kWriterThreads) void quantize_k_groupwise_int4_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, uint16_t* __restrict__ scale,
@@ -163,48 +190,22 @@ __global__ __launch_bounds__(kWriterThreads) void quantize_k_groupwise_int4_kern
         const int t = min(t_start + row + 16 * i, t_end - 1);   // in bounds; duplicates do not move the max
         raw[i] = stream16(x + (base + t) * 128 + 8 * c);
     }
-    uint32_t amax[8];   // NaN-propagating absmax per channel, as bits
+    uint32_t m[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) amax[e] = 0u;
+    for (int i = 0; i < TPR; ++i)
 #pragma unroll
-    for (int i = 0; i < TPR; ++i) {
-        float xf[8];
-        f16x8_to_f32(raw[i], xf);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) amax[e] = max(amax[e], abs_bits(xf[e]));
-    }
-
-    __shared__ uint32_t s_max[16][128];
-    __shared__ float s_scale[128];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s_max[row][8 * c + e] = amax[e];
-    __syncthreads();
-    if (threadIdx.x < 128) {
-        uint32_t m = 0u;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) m = max(m, s_max[r][threadIdx.x]);
-        const float sc = sym_scale(m, 7.0f);
-        s_scale[threadIdx.x] = sc;
-        scale[sslot * 128 + threadIdx.x] = f2h_bits(sc);
-    }
-    __syncthreads();
-
-    float sv[8], rcp[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        sv[e] = s_scale[8 * c + e];
-        rcp[e] = recip_approx(sv[e]);
-    }
+        for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], raw[i][d]);
+    __shared__ __attribute__((aligned(16))) KScales lds;
+    float sv[8], rv[8];
+    k_group_scales(lds, m, scale + sslot * 128, sv, rv);
 #pragma unroll
     for (int i = 0; i < TPR; ++i) {
         const int t = t_start + row + 16 * i;
-        float xf[8];
-        f16x8_to_f32(raw[i], xf);
-        uint32_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w |= (uint32_t)(sym_code(xf[e], sv[e], rcp[e], 7) & 0xF) << (4 * e);
+        const uint32_t w[4] = {raw[i][0], raw[i][1], raw[i][2], raw[i][3]};
+        uint32_t code[8];
+        code_words<7>(w, sv, rv, code);
         if (t < t_end)
-            __builtin_nontemporal_store(w, reinterpret_cast<uint32_t*>(q + (qbase + t) * 64 + 4 * c));
+            __builtin_nontemporal_store(pack_nibbles(code), reinterpret_cast<uint32_t*>(q + (qbase + t) * 64 + 4 * c));
     }
 }
 
@@ -224,44 +225,21 @@ __global__ __launch_bounds__(kWriterThreads) void quantize_k_groupwise_int4_larg
     const long qbase = bh * map.dst_len + map.dst_off;      // cache row of token 0
     const long sslot = bh * dst_groups + map.dst_off / group_size + g;
 
-    uint32_t amax[8];   // NaN-propagating absmax per channel, as bits
-#pragma unroll
-    for (int e = 0; e < 8; ++e) amax[e] = 0u;
+    uint32_t m[4] = {0u, 0u, 0u, 0u};
     for (int t = t_start + row; t < t_end; t += 16) {
-        float xf[8];
-        f16x8_to_f32(load16(x + (base + t) * 128 + 8 * c), xf);
+        const u32x4 v = load16(x + (base + t) * 128 + 8 * c);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) amax[e] = max(amax[e], abs_bits(xf[e]));
+        for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], v[d]);
     }
-
-    __shared__ uint32_t s_max[16][128];
-    __shared__ float s_scale[128];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s_max[row][8 * c + e] = amax[e];
-    __syncthreads();
-    if (threadIdx.x < 128) {
-        uint32_t m = 0u;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) m = max(m, s_max[r][threadIdx.x]);
-        const float sc = sym_scale(m, 7.0f);
-        s_scale[threadIdx.x] = sc;
-        scale[sslot * 128 + threadIdx.x] = f2h_bits(sc);
-    }
-    __syncthreads();
-
-    float sv[8], rcp[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        sv[e] = s_scale[8 * c + e];
-        rcp[e] = recip_approx(sv[e]);
-    }
+    __shared__ __attribute__((aligned(16))) KScales lds;
+    float sv[8], rv[8];
+    k_group_scales(lds, m, scale + sslot * 128, sv, rv);
     for (int t = t_start + row; t < t_end; t += 16) {
-        float xf[8];
-        f16x8_to_f32(load16(x + (base + t) * 128 + 8 * c), xf);
-        uint32_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w |= (uint32_t)(sym_code(xf[e], sv[e], rcp[e], 7) & 0xF) << (4 * e);
-        *reinterpret_cast<uint32_t*>(q + (qbase + t) * 64 + 4 * c) = w;
+        const u32x4 v = load16(x + (base + t) * 128 + 8 * c);
+        const uint32_t w[4] = {v[0], v[1], v[2], v[3]};
+        uint32_t code[8];
+        code_words<7>(w, sv, rv, code);
+        *reinterpret_cast<uint32_t*>(q + (qbase + t) * 64 + 4 * c) = pack_nibbles(code);
     }
 }
 
@@ -309,7 +287,7 @@ int launch_quantize_k_groupwise_int4(const void* x, void* q, void* scale, int ro
     else if (group_size <= 64)
         hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<4>, grid, blk, 0, stream, xp, qp, sp, group_size, map, dst_groups);
     else if (group_size <= 128)
-        hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<8>, grid, blk, 0, stream, xp, qp, sp, group_size, map, dst_groups);
+        hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<8>, grid, blk, kWideGroupLds, stream, xp, qp, sp, group_size, map, dst_groups);
     else
         hipLaunchKernelGGL(quantize_k_groupwise_int4_large_kernel, grid, blk, 0, stream, xp, qp, sp, group_size, map, dst_groups);
     return check_launch();
@@ -346,62 +324,37 @@ __global__ __launch_bounds__(kWriterThreads) void kivi_append_token_kernel(
     }
     if (row == (r & 15)) *reinterpret_cast<u32x4*>(kopen + (long)r * 128) = knew;
 
-    uint32_t amax[8];   // NaN-propagating absmax per channel, as bits
+    uint32_t m[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) amax[e] = 0u;
+    for (int i = 0; i < TPR; ++i)
 #pragma unroll
-    for (int i = 0; i < TPR; ++i) {
-        float xf[8];
-        f16x8_to_f32(raw[i], xf);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) amax[e] = max(amax[e], abs_bits(xf[e]));
-    }
-    __shared__ uint32_t s_max[16][128];
-    __shared__ float s_scale[128];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s_max[row][8 * c + e] = amax[e];
-    __syncthreads();
+        for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], raw[i][d]);
     const int start = pos - r;
-    if (threadIdx.x < 128) {
-        uint32_t m = 0u;
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) m = max(m, s_max[rr][threadIdx.x]);
-        const float sc = sym_scale(m, 7.0f);
-        s_scale[threadIdx.x] = sc;
-        k_scale[(bh * n_groups + start / group_size) * 128 + threadIdx.x] = f2h_bits(sc);
-    }
-    __syncthreads();
-    float sv[8], rcp[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        sv[e] = s_scale[8 * c + e];
-        rcp[e] = recip_approx(sv[e]);
-    }
+    __shared__ __attribute__((aligned(16))) KScales lds;
+    float sv[8], rv[8];
+    k_group_scales(lds, m, k_scale + (bh * n_groups + start / group_size) * 128, sv, rv);
 #pragma unroll
     for (int i = 0; i < TPR; ++i) {
         const int t = row + 16 * i;
-        float xf[8];
-        f16x8_to_f32(raw[i], xf);
-        uint32_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w |= (uint32_t)(sym_code(xf[e], sv[e], rcp[e], 7) & 0xF) << (4 * e);
-        if (t <= r) *reinterpret_cast<uint32_t*>(k_q + (bh * max_len + start + t) * 64 + 4 * c) = w;
+        const uint32_t w[4] = {raw[i][0], raw[i][1], raw[i][2], raw[i][3]};
+        uint32_t code[8];
+        code_words<7>(w, sv, rv, code);
+        if (t <= r) *reinterpret_cast<uint32_t*>(k_q + (bh * max_len + start + t) * 64 + 4 * c) = pack_nibbles(code);
     }
 
     // ---- V: the token per token (row 0's 16 lanes)
     if (row == 0) {
-        float xf[8];
-        f16x8_to_f32(load16(v_in + bh * v_stride + 8 * c), xf);
-        uint32_t amax1 = 0u;
+        const u32x4 vr = load16(v_in + bh * v_stride + 8 * c);
+        const uint32_t w[4] = {vr[0], vr[1], vr[2], vr[3]};
+        uint32_t mv = 0u;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) amax1 = max(amax1, abs_bits(xf[e]));
-        amax1 = row16_umax(amax1);
-        const float sc = sym_scale(amax1, 7.0f);
-        const float rc = recip_approx(sc);
-        uint32_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w |= (uint32_t)(sym_code(xf[e], sc, rc, 7) & 0xF) << (4 * e);
-        *reinterpret_cast<uint32_t*>(v_q + (bh * max_len + pos) * 64 + 4 * c) = w;
+        for (int d = 0; d < 4; ++d) mv = max_abs2(mv, w[d]);
+        const uint32_t amax16 = row16_umax(max(mv & 0xFFFFu, mv >> 16));
+        const float sc = sym_scale(__float_as_uint(h2f((uint16_t)amax16)), 7.0f);
+        const float s1[1] = {sc}, r1[1] = {recip_approx(sc)};
+        uint32_t code[8];
+        code_words<7>(w, s1, r1, code);
+        *reinterpret_cast<uint32_t*>(v_q + (bh * max_len + pos) * 64 + 4 * c) = pack_nibbles(code);
         if (c == 0) v_scale[bh * max_len + pos] = f2h_bits(sc);
     }
 }
