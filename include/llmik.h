@@ -227,6 +227,23 @@ LLMIK_API llmik_status llmik_kivi_append_token_int4(
     void* v_scale, int batch, int n_kv_heads, int head_dim, int max_len, int group_size, int length,
     void* stream);
 
+/* n decode or prefill tokens appended to a KIVI INT4 cache holding `length`
+ * tokens, and / or the cache's fp16 view, in one launch (two where the call
+ * completes an open group and opens another): the launches of
+ * Int4KIVICache.append for n tokens, the same stored bits, and the
+ * reference's dequantised view (integration/kv_int4_cache.py:225-245): fp16
+ * code * scale of the full groups, the fp16 tokens of the open one.
+ *   k, v     [batch, n_kv_heads, k_len / v_len, 128] fp16, tokens 0 .. n - 1
+ *            (may be null when n is 0)
+ *   k_open   as above; v_open the same for V, or null (no view then)
+ *   k_view, v_view [batch, n_kv_heads, length + n, 128] fp16, or both null
+ * The other tensors are llmik_kivi_append_token_int4's. group_size <= 128;
+ * length + n <= max_len. */
+LLMIK_API llmik_status llmik_kivi_append_int4(
+    const void* k, int k_len, const void* v, int v_len, void* k_open, void* v_open, void* k_q, void* k_scale,
+    void* v_q, void* v_scale, void* k_view, void* v_view, int batch, int n_kv_heads, int head_dim, int n,
+    int max_len, int group_size, int length, void* stream);
+
 /* -------------------------------------------------------------------- W4A16
  * out[M, N] = act[M, K] @ dequant(W)[K, N], W[k, n] = q[k, n] * scale[k/g, n],
  * fp32 accumulation.

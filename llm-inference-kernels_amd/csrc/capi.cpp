@@ -291,6 +291,29 @@ LLMIK_API llmik_status llmik_kivi_append_token_int4(
                                     max_len, n_groups, as_stream(stream));
 }
 
+LLMIK_API llmik_status llmik_kivi_append_int4(
+    const void* k, int k_len, const void* v, int v_len, void* k_open, void* v_open, void* k_q, void* k_scale,
+    void* v_q, void* v_scale, void* k_view, void* v_view, int batch, int n_kv_heads, int head_dim, int n,
+    int max_len, int group_size, int length, void* stream) {
+    if (batch < 0 || n_kv_heads < 0 || n < 0 || max_len < 0 || length < 0) return invalid("negative dimension");
+    if (head_dim != 128) return invalid("only head_dim=128 supported");
+    if (group_size <= 0 || group_size > 128) return invalid("group_size must be in 1..128");
+    if ((long)length + n > max_len) return invalid("length + n exceeds the cache length");
+    if (n > 0 && (n > k_len || n > v_len)) return invalid("n exceeds the token length of k or v");
+    if ((k_view == nullptr) != (v_view == nullptr)) return invalid("k_view and v_view go together");
+    if ((long)batch * n_kv_heads > 65535L) return invalid("batch * n_kv_heads exceeds 65535");
+    if ((long)batch * n_kv_heads > 0 && ((n > 0 && (!k || !v)) || !k_open || (k_view && !v_open) || !k_q ||
+                                         !k_scale || !v_q || !v_scale))
+        return invalid("null pointer");
+    if (!aligned(k, 16) || !aligned(v, 16) || !aligned(k_open, 16) || !aligned(v_open, 16) || !aligned(k_view, 16) ||
+        !aligned(v_view, 16) || !aligned(k_q, 4) || !aligned(v_q, 4) || !aligned(k_scale, 16) || !aligned(v_scale, 2))
+        return set_error(LLMIK_ERR_ALIGNMENT, "fp16 tokens, views and k_scale must be 16-byte aligned");
+    const int n_groups = (max_len + group_size - 1) / group_size;
+    return launch_kivi_append(k, (long)k_len * 128, v, (long)v_len * 128, k_open, v_open, k_q, k_scale, v_q, v_scale,
+                              k_view, v_view, batch * n_kv_heads, n, length, group_size, max_len, n_groups,
+                              as_stream(stream));
+}
+
 namespace {
 int check_gemm(const void* act, const void* w, const void* scale, const void* out, int M, int N,
                int K, int group_size) {

@@ -232,11 +232,10 @@ __device__ __forceinline__ float quant_round(float x, float s, float r) {
 __device__ __forceinline__ float recip_approx(float s) { return __builtin_amdgcn_rcpf(s); }
 
 // ---- torch's non-finite semantics for the symmetric quantisers ------------
-// |x| as bits. With the sign cleared, the unsigned order of the bit patterns
-// is the float order and every NaN sits above +inf, so an unsigned max over
-// them is torch's `x.abs().amax()`, which propagates NaN (fmaxf drops it).
-__device__ __forceinline__ uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7FFFFFFFu; }
-
+// Absolute values are compared as bits: with the sign cleared, the unsigned
+// order of the bit patterns is the float order and every NaN sits above +inf,
+// so an unsigned max over them is torch's `x.abs().amax()`, which propagates
+// NaN (fmaxf drops it).
 // Unsigned max over the 16 lanes of a DPP row; every lane gets the result.
 __device__ __forceinline__ uint32_t row16_umax(uint32_t v) {
     v = max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kDppQuadXor1, 0xF, 0xF, true));

@@ -123,24 +123,36 @@ __global__ __launch_bounds__(kWriterThreads) void quantize_per_token_kernel(
     }
 }
 
-// The K writers' workgroup: 16 rows of 16 lanes, lane c of a row owning
-// channels 8c..8c+7. Merges the rows' packed absmax (fp16 bit patterns, m) in
-// LDS, computes the 128 channels' scales and their reciprocals once, stores
-// the fp16 scales and hands each lane its channels'.
+// The K writers' workgroup: NT / 16 rows of 16 lanes, lane c of a row owning
+// channels 8c..8c+7. Merges the rows' packed absmax (fp16 bit patterns, m):
+// the four rows of a wave by lane swaps, the waves through LDS; computes the
+// 128 channels' scales and their reciprocals once, stores the fp16 scales and
+// hands each lane its channels'.
+template <int NT>
 struct KScales {
-    uint16_t maxes[16][128];
+    uint16_t maxes[NT / kWave][128];
     float scale[128], rcp[128];
 };
-__device__ __forceinline__ void k_group_scales(KScales& l, const uint32_t (&m)[4], uint16_t* __restrict__ scale,
+template <int NT>
+__device__ __forceinline__ void k_group_scales(KScales<NT>& l, uint32_t (&m)[4], uint16_t* __restrict__ scale,
                                                float (&sv)[8], float (&rv)[8]) {
-    const int row = threadIdx.x >> 4;
+    const int lane = threadIdx.x & (kWave - 1);
     const int c = threadIdx.x & 15;
-    *reinterpret_cast<u32x4*>(&l.maxes[row][8 * c]) = u32x4{m[0], m[1], m[2], m[3]};
+    // Two copies of a value swap their 32-lane halves (16-lane rows): the two
+    // results hold each half (row) in both places.
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const auto h = __builtin_amdgcn_permlane32_swap(m[d], m[d], false, false);
+        m[d] = max_abs2(h[0], h[1]);
+        const auto r = __builtin_amdgcn_permlane16_swap(m[d], m[d], false, false);
+        m[d] = max_abs2(r[0], r[1]);
+    }
+    if (lane < 16) *reinterpret_cast<u32x4*>(&l.maxes[threadIdx.x / kWave][8 * c]) = u32x4{m[0], m[1], m[2], m[3]};
     __syncthreads();
     if (threadIdx.x < 128) {
         uint32_t a = 0u;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) a = max(a, (uint32_t)l.maxes[r][threadIdx.x]);
+        for (int r = 0; r < NT / kWave; ++r) a = max(a, (uint32_t)l.maxes[r][threadIdx.x]);
         const float sc = sym_scale(__float_as_uint(h2f((uint16_t)a)), 7.0f);
         l.scale[threadIdx.x] = sc;
         l.rcp[threadIdx.x] = recip_approx(sc);
@@ -155,8 +167,8 @@ __device__ __forceinline__ void k_group_scales(KScales& l, const uint32_t (&m)[4
 }
 
 // Dynamic LDS that, beside the static part, admits four workgroups to a CU's 160 KiB.
-constexpr size_t kWideGroupLds = 36 * 1024 - sizeof(KScales);
-static_assert(5 * (kWideGroupLds + sizeof(KScales)) > 160 * 1024 && 4 * (kWideGroupLds + sizeof(KScales)) <= 160 * 1024,
+constexpr size_t kWideGroupLds = 36 * 1024 - sizeof(KScales<kWriterThreads>);
+static_assert(5 * (kWideGroupLds + sizeof(KScales<kWriterThreads>)) > 160 * 1024 && 4 * (kWideGroupLds + sizeof(KScales<kWriterThreads>)) <= 160 * 1024,
               "four workgroups, not five");
 
 // K per channel, group-wise: one workgroup per (batch, kv_head, group). Row r
@@ -195,7 +207,7 @@ __global__ __launch_bounds__(kWriterThreads) void quantize_k_groupwise_int4_kern
     for (int i = 0; i < TPR; ++i)
 #pragma unroll
         for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], raw[i][d]);
-    __shared__ __attribute__((aligned(16))) KScales lds;
+    __shared__ __attribute__((aligned(16))) KScales<kWriterThreads> lds;
     float sv[8], rv[8];
     k_group_scales(lds, m, scale + sslot * 128, sv, rv);
 #pragma unroll
@@ -231,7 +243,7 @@ __global__ __launch_bounds__(kWriterThreads) void quantize_k_groupwise_int4_larg
 #pragma unroll
         for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], v[d]);
     }
-    __shared__ __attribute__((aligned(16))) KScales lds;
+    __shared__ __attribute__((aligned(16))) KScales<kWriterThreads> lds;
     float sv[8], rv[8];
     k_group_scales(lds, m, scale + sslot * 128, sv, rv);
     for (int t = t_start + row; t < t_end; t += 16) {
@@ -330,7 +342,7 @@ __global__ __launch_bounds__(kWriterThreads) void kivi_append_token_kernel(
 #pragma unroll
         for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], raw[i][d]);
     const int start = pos - r;
-    __shared__ __attribute__((aligned(16))) KScales lds;
+    __shared__ __attribute__((aligned(16))) KScales<kWriterThreads> lds;
     float sv[8], rv[8];
     k_group_scales(lds, m, k_scale + (bh * n_groups + start / group_size) * 128, sv, rv);
 #pragma unroll
@@ -376,6 +388,230 @@ int launch_kivi_append_token(const void* k, long k_stride, const void* v, long v
     else if (tpr <= 2) go(std::integral_constant<int, 2>{});
     else if (tpr <= 4) go(std::integral_constant<int, 4>{});
     else go(std::integral_constant<int, 8>{});
+    return check_launch();
+}
+
+// Several tokens appended to a KIVI INT4 cache, and / or its fp16 view, one
+// workgroup per (group of group_size tokens, (batch, kv_head) row). Replaces
+// the V writer, the K writer of the whole groups, a copy of the open group and
+// the K writer of the open group (four launches), and for the view unpacking,
+// scaling and concatenating in torch (about 20 launches over 32-bit
+// intermediates). A group's tokens are loaded once, K and V together:
+//   * a group that gains tokens: K scale and codes over all its tokens (the
+//     ones before `start` from k_open), V codes and scales of its new tokens;
+//     its new K tokens go to k_open if it began before `start` or stays open,
+//     its new V tokens to v_open if it stays open;
+//   * view: fp16(code * scale) of a full group, the fp16 tokens of an open one
+//     (the old ones from k_open / v_open); full groups before `start` are
+//     read from the codes.
+// k_open and v_open hold one group, so a launch that reads the tokens of a
+// group begun before `start` must not also open another (launch_kivi_append
+// splits the call there). Bound by the read + write stream (append of 3000
+// tokens, B=4 Hkv=8 g32: 62 MB, 4.6 TB/s); us, before -> now: that append 21.9
+// -> 13.5, B=8 n=4096 g128 33.8 -> 30.4, B=1 n=50 g32 9.8 -> 3.3; with the
+// view, eager, B=1 n=2048 g32: 176-192 -> 7.8.
+struct KiviAppend {
+    const uint16_t* k;   // token t of row bh: k + bh * k_stride + (t - start) * 128
+    const uint16_t* v;
+    long k_stride, v_stride;
+    uint16_t* k_open;    // [rows, group_size, 128]
+    uint16_t* v_open;    // as k_open, or null
+    int8_t* k_q;         // [rows, max_len, 64]
+    uint16_t* k_scale;   // [rows, n_groups, 128]
+    int8_t* v_q;
+    uint16_t* v_scale;   // [rows, max_len]
+    uint16_t* k_view;    // [rows, view_len, 128], or null
+    uint16_t* v_view;
+    int start, end;      // live length before and after
+    int group0;          // group of workgroup 0
+    int group_size, max_len, n_groups, view_len;
+};
+
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+    return (uint32_t)f2h_bits(a) | ((uint32_t)f2h_bits(b) << 16);
+}
+
+template <int NT, int TPR, bool VIEW>
+__global__ __launch_bounds__(NT) void kivi_append_kernel(KiviAppend p) {
+    constexpr int kRows = NT / 16;   // token rows of the workgroup; kRows * TPR >= group_size
+    const int grp = p.group0 + blockIdx.x;
+    const long bh = blockIdx.y;
+    const int row = threadIdx.x >> 4;
+    const int c = threadIdx.x & 15;
+    const int t0 = grp * p.group_size;
+    const int t1 = min(t0 + p.group_size, p.end);   // t0 < end: the group has a token
+    const bool full = t1 - t0 == p.group_size;
+    const long qrow = bh * p.max_len;
+    uint16_t* const sc_row = p.k_scale + (bh * p.n_groups + grp) * 128;
+    uint16_t* const kopen = p.k_open + bh * (long)p.group_size * 128 + 8 * c;
+    uint16_t* const vopen = (p.v_open ? p.v_open : p.k_open) + bh * (long)p.group_size * 128 + 8 * c;
+
+    if (VIEW && full && t1 <= p.start) {   // a full group of the past: from its codes
+        float sv[8];
+        f16x8_to_f32(load16(sc_row + 8 * c), sv);
+#pragma unroll
+        for (int i = 0; i < TPR; ++i) {
+            const int t = t0 + row + kRows * i;
+            if (t >= t1) break;
+            float kc[8], vc[8];
+            i4x8_to_f32(load4(p.k_q + (qrow + t) * 64 + 4 * c), kc);
+            i4x8_to_f32(load4(p.v_q + (qrow + t) * 64 + 4 * c), vc);
+            const float vs = h2f(p.v_scale[qrow + t]);
+            u32x4 ko, vo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                ko[e] = pack_f16(kc[2 * e] * sv[2 * e], kc[2 * e + 1] * sv[2 * e + 1]);
+                vo[e] = pack_f16(vc[2 * e] * vs, vc[2 * e + 1] * vs);
+            }
+            const long o = (bh * p.view_len + t) * 128 + 8 * c;
+            *reinterpret_cast<u32x4*>(p.k_view + o) = ko;
+            *reinterpret_cast<u32x4*>(p.v_view + o) = vo;
+        }
+        return;
+    }
+
+    // Tokens of this lane's row; past the group's end its last one again
+    // (in bounds, does not move the maximum, nothing of it is stored).
+    u32x4 kr[TPR], vr[TPR];
+#pragma unroll
+    for (int i = 0; i < TPR; ++i) {
+        const int t = min(t0 + row + kRows * i, t1 - 1);
+        const bool fresh = t >= p.start;
+        kr[i] = fresh ? stream16(p.k + bh * p.k_stride + (long)(t - p.start) * 128 + 8 * c)
+                      : load16(kopen + (long)(t - t0) * 128);
+        // An old token's V is wanted for the view only.
+        vr[i] = fresh ? stream16(p.v + bh * p.v_stride + (long)(t - p.start) * 128 + 8 * c)
+                      : (VIEW ? load16(vopen + (long)(t - t0) * 128) : u32x4{0u, 0u, 0u, 0u});
+    }
+    if (VIEW && t1 <= p.start) {   // the open group, unchanged
+#pragma unroll
+        for (int i = 0; i < TPR; ++i) {
+            const int t = t0 + row + kRows * i;
+            if (t >= t1) break;
+            const long o = (bh * p.view_len + t) * 128 + 8 * c;
+            *reinterpret_cast<u32x4*>(p.k_view + o) = kr[i];
+            *reinterpret_cast<u32x4*>(p.v_view + o) = vr[i];
+        }
+        return;
+    }
+
+    uint32_t m[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < TPR; ++i)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) m[d] = max_abs2(m[d], kr[i][d]);
+    __shared__ __attribute__((aligned(16))) KScales<NT> lds;
+    float sv[8], rv[8];
+    k_group_scales(lds, m, sc_row, sv, rv);
+#pragma unroll
+    for (int i = 0; i < TPR; ++i) {
+        const int t = t0 + row + kRows * i;
+        const bool ok = t < t1, fresh = ok && t >= p.start;
+        const uint32_t kw[4] = {kr[i][0], kr[i][1], kr[i][2], kr[i][3]};
+        uint32_t kc[8];
+        code_words<7>(kw, sv, rv, kc);
+        const uint32_t vw[4] = {vr[i][0], vr[i][1], vr[i][2], vr[i][3]};
+        uint32_t mv = 0u;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) mv = max_abs2(mv, vw[d]);
+        const float vs = sym_scale(__float_as_uint(h2f((uint16_t)row16_umax(max(mv & 0xFFFFu, mv >> 16)))), 7.0f);
+        const float s1[1] = {vs}, r1[1] = {recip_approx(vs)};
+        uint32_t vc[8];
+        code_words<7>(vw, s1, r1, vc);
+        if (ok) __builtin_nontemporal_store(pack_nibbles(kc), reinterpret_cast<uint32_t*>(p.k_q + (qrow + t) * 64 + 4 * c));
+        if (fresh) {
+            __builtin_nontemporal_store(pack_nibbles(vc), reinterpret_cast<uint32_t*>(p.v_q + (qrow + t) * 64 + 4 * c));
+            if (c == 0) p.v_scale[qrow + t] = f2h_bits(vs);
+            if (t0 < p.start || !full) *reinterpret_cast<u32x4*>(kopen + (long)(t - t0) * 128) = kr[i];
+            if (p.v_open && !full) *reinterpret_cast<u32x4*>(vopen + (long)(t - t0) * 128) = vr[i];
+        }
+        if constexpr (VIEW) {
+            if (ok) {
+                u32x4 ko = kr[i], vo = vr[i];
+                if (full) {
+                    // The code as a float is its word minus kCodeMagic, except
+                    // that a NaN word stands for code 0; fp16(code * scale) is
+                    // NaN in both, as that word's scale is NaN or inf.
+                    const float v16 = h2f(f2h_bits(vs));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float kf[2], vf[2];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            kf[u] = (__uint_as_float(kc[2 * e + u]) - kCodeMagic) * h2f(f2h_bits(sv[2 * e + u]));
+                            vf[u] = (__uint_as_float(vc[2 * e + u]) - kCodeMagic) * v16;
+                        }
+                        ko[e] = pack_f16(kf[0], kf[1]);
+                        vo[e] = pack_f16(vf[0], vf[1]);
+                    }
+                }
+                const long o = (bh * p.view_len + t) * 128 + 8 * c;
+                *reinterpret_cast<u32x4*>(p.k_view + o) = ko;
+                *reinterpret_cast<u32x4*>(p.v_view + o) = vo;
+            }
+        }
+    }
+}
+
+int launch_kivi_append(const void* k, long k_stride, const void* v, long v_stride, void* k_open, void* v_open,
+                       void* k_q, void* k_scale, void* v_q, void* v_scale, void* k_view, void* v_view, int rows,
+                       int n, int length, int group_size, int max_len, int n_groups, hipStream_t stream) {
+    if (rows == 0 || length + n == 0) return LLMIK_OK;
+    if (rows > 65535) return set_error(LLMIK_ERR_UNSUPPORTED, "batch * n_kv_heads exceeds 65535");
+    const bool view = k_view != nullptr;
+    if (n == 0 && !view) return LLMIK_OK;
+    KiviAppend p{};
+    p.k = static_cast<const uint16_t*>(k);
+    p.v = static_cast<const uint16_t*>(v);
+    p.k_stride = k_stride;
+    p.v_stride = v_stride;
+    p.k_open = static_cast<uint16_t*>(k_open);
+    p.v_open = static_cast<uint16_t*>(v_open);
+    p.k_q = static_cast<int8_t*>(k_q);
+    p.k_scale = static_cast<uint16_t*>(k_scale);
+    p.v_q = static_cast<int8_t*>(v_q);
+    p.v_scale = static_cast<uint16_t*>(v_scale);
+    p.k_view = static_cast<uint16_t*>(k_view);
+    p.v_view = static_cast<uint16_t*>(v_view);
+    p.group_size = group_size;
+    p.max_len = max_len;
+    p.n_groups = n_groups;
+    p.view_len = length + n;
+    // Groups [first, the group of end - 1].
+    auto go = [&](int first, int start, int end) {
+        p.group0 = first;
+        p.start = start;
+        p.end = end;
+        const dim3 grid((end - 1) / group_size - first + 1, rows);
+        auto with = [&](auto nt, auto tpr) {
+            constexpr int NT = decltype(nt)::value, T = decltype(tpr)::value;
+            if (view) hipLaunchKernelGGL((kivi_append_kernel<NT, T, true>), grid, dim3(NT), 0, stream, p);
+            else hipLaunchKernelGGL((kivi_append_kernel<NT, T, false>), grid, dim3(NT), 0, stream, p);
+        };
+        using std::integral_constant;
+        // Threads x tokens per lane (us): g32 B=4 n=3000 256 x 2 13.5, 512 x 1
+        // 14.0, 128 x 4 15.2; g64 B=2 n=10000 512 x 2 19.8, 256 x 4 21.2; g128
+        // B=8 n=4096 512 x 4 30.4, 256 x 8 33.8, 1024 x 2 39.9, but with at
+        // most one workgroup per CU (B=1 n=2048) 6.75, 9.8 and 5.9.
+        if (group_size <= 16) with(integral_constant<int, 256>{}, integral_constant<int, 1>{});
+        else if (group_size <= 32) with(integral_constant<int, 256>{}, integral_constant<int, 2>{});
+        else if (group_size <= 64) with(integral_constant<int, 512>{}, integral_constant<int, 2>{});
+        else if ((long)grid.x * rows > device_cu_count()) with(integral_constant<int, 512>{}, integral_constant<int, 4>{});
+        else with(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
+    };
+    const int first = view ? 0 : length / group_size;
+    const int boundary = (length / group_size + 1) * group_size;   // end of the group begun before `length`
+    const int end = length + n;
+    if (length % group_size != 0 && end > boundary && end % group_size != 0) {
+        // The open group is completed and another one opened: k_open / v_open
+        // are read by the first launch and rewritten by the second.
+        go(first, length, boundary);
+        p.k += (long)(boundary - length) * 128;
+        p.v += (long)(boundary - length) * 128;
+        go(boundary / group_size, boundary, end);
+    } else {
+        go(first, length, end);
+    }
     return check_launch();
 }
 

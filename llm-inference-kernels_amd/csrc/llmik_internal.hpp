@@ -79,6 +79,12 @@ int launch_kivi_append_token(const void* k, long k_stride, const void* v, long v
                              void* k_q, void* k_scale, void* v_q, void* v_scale, int rows, int r,
                              int pos, int group_size, int max_len, int n_groups, hipStream_t stream);
 
+// n tokens appended at `length` and / or (k_view non-null) the fp16 view of all
+// length + n; v_open may be null without a view.
+int launch_kivi_append(const void* k, long k_stride, const void* v, long v_stride, void* k_open, void* v_open,
+                       void* k_q, void* k_scale, void* v_q, void* v_scale, void* k_view, void* v_view, int rows,
+                       int n, int length, int group_size, int max_len, int n_groups, hipStream_t stream);
+
 // ---- W4A16 -----------------------------------------------------------------
 struct GemmPlan {
     int kind;          // 0: single-row VALU GEMV, 1: tiled multi-row VALU,

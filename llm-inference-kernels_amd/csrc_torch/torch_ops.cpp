@@ -16,8 +16,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <climits>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <utility>
 #include <vector>
 
@@ -335,6 +337,78 @@ void kivi_append_token_int4(const Tensor& k, const Tensor& v, const Tensor& k_op
                                        stream_of(k)));
 }
 
+// Token stride of x's rows as token_rows gives it, or 0 where it raises.
+int64_t token_rows_or_zero(const Tensor& x) {
+    const int64_t batch = x.size(0), heads = x.size(1), n = x.size(2), d = x.size(3);
+    if (x.stride(3) != 1 || (n > 1 && x.stride(2) != d)) return 0;
+    int64_t row = n * d;
+    if (heads > 1) {
+        row = x.stride(1);
+        if (batch > 1 && x.stride(0) != heads * row) return 0;
+    } else if (batch > 1) {
+        row = x.stride(0);
+    }
+    return (row % d == 0 && row >= n * d) ? row / d : 0;
+}
+
+// Several tokens appended to a KIVI INT4 cache of `length` tokens in one launch
+// and, with v_open, the fp16 view of the whole cache: (k, v) views, or (None,
+// None) without v_open. k and v may be None (the view alone). Returns None
+// where the launch does not take the call (a head_dim other than 128, groups
+// above 128, rows that are not equally spaced or not 16-byte aligned): the
+// caller's general path then serves or refuses it. The cache tensors are the
+// cache object's own; its shapes are re-checked here because the kernel
+// trusts them.
+py::object kivi_append_int4(const std::optional<Tensor>& k, const std::optional<Tensor>& v, const Tensor& k_open,
+                            const std::optional<Tensor>& v_open, const Tensor& k_q, const Tensor& k_scale,
+                            const Tensor& v_q, const Tensor& v_scale, int64_t length, int64_t group_size) {
+    if (group_size <= 0 || group_size > 128 || k_q.dim() != 4 || k_q.size(3) != 64 || !k_q.is_cuda()) return py::none();
+    const int64_t b = k_q.size(0), h = k_q.size(1), max_len = k_q.size(2);
+    const int64_t groups = (max_len + group_size - 1) / group_size;
+    if (k_q.scalar_type() != at::kChar || v_q.scalar_type() != at::kChar || k_scale.scalar_type() != at::kHalf ||
+        v_scale.scalar_type() != at::kHalf || k_open.scalar_type() != at::kHalf || v_q.sizes() != k_q.sizes() ||
+        k_scale.sizes() != at::IntArrayRef({b, h, groups, 128}) || v_scale.sizes() != at::IntArrayRef({b, h, max_len}) ||
+        k_open.sizes() != at::IntArrayRef({b, h, group_size, 128}) || b * h > 65535)
+        return py::none();
+    int64_t n = 0, k_len = 0, v_len = 0;
+    std::vector<Tensor> all{k_open, k_q, k_scale, v_q, v_scale};
+    if (v_open.has_value()) {
+        if (v_open->scalar_type() != at::kHalf || v_open->sizes() != k_open.sizes()) return py::none();
+        all.push_back(*v_open);
+    }
+    for (const Tensor& t : all)
+        if (!t.is_contiguous()) return py::none();
+    if (k.has_value() != v.has_value()) return py::none();
+    if (k.has_value()) {
+        for (const Tensor* x : {&*k, &*v})
+            if (x->scalar_type() != at::kHalf || x->dim() != 4 || x->size(0) != b || x->size(1) != h ||
+                x->size(3) != 128 || x->size(2) != k->size(2))
+                return py::none();
+        n = k->size(2);
+        k_len = token_rows_or_zero(*k);
+        v_len = token_rows_or_zero(*v);
+        if (n > 0 && (k_len == 0 || v_len == 0 || k_len > INT_MAX || v_len > INT_MAX)) return py::none();
+        all.push_back(*k);
+        all.push_back(*v);
+    }
+    for (const Tensor& t : all)
+        if (t.device() != k_q.device() || (uintptr_t)t.data_ptr() % 16 != 0) return py::none();
+    if (length < 0 || length + n > max_len) return py::none();
+    const c10::DeviceGuard guard(k_q.device());
+    Tensor kv, vv;
+    if (v_open.has_value()) {
+        kv = at::empty({b, h, length + n, 128}, k_open.options());
+        vv = at::empty({b, h, length + n, 128}, k_open.options());
+    }
+    check(llmik_kivi_append_int4(k ? ptr(*k) : nullptr, (int)k_len, v ? ptr(*v) : nullptr, (int)v_len, ptr(k_open),
+                                 v_open ? ptr(*v_open) : nullptr, ptr(k_q), ptr(k_scale), ptr(v_q), ptr(v_scale),
+                                 v_open && kv.numel() ? ptr(kv) : nullptr, v_open && kv.numel() ? ptr(vv) : nullptr,
+                                 (int)b, (int)h, 128, (int)n, (int)max_len, (int)group_size, (int)length,
+                                 stream_of(k_q)));
+    if (!v_open.has_value()) return py::make_tuple(py::none(), py::none());
+    return py::make_tuple(kv, vv);
+}
+
 // -------------------------------------------------------------------- W4A16
 
 Tensor gemm(const Tensor& act, const Tensor& weight_packed, const Tensor& scale, int64_t group_size, bool f32) {
@@ -567,6 +641,7 @@ PYBIND11_MODULE(_C, m) {
     m.def("quantize_v_per_token_int4_into", &quantize_v_per_token_int4_into);
     m.def("quantize_k_per_channel_groupwise_int4_into", &quantize_k_per_channel_groupwise_int4_into);
     m.def("kivi_append_token_int4", &kivi_append_token_int4);
+    m.def("kivi_append_int4", &kivi_append_int4);
     m.def("w4a16_gemm", &w4a16_gemm);
     m.def("w4a16_gemm_f32out", &w4a16_gemm_f32out);
     m.def("w4a16_gemm_swiglu", &w4a16_gemm_swiglu);

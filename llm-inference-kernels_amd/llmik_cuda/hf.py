@@ -203,7 +203,12 @@ class KIVILayer(CacheLayerMixin):
         c, g = self.cache, self.group_size
         n = key_states.shape[-2]
         start = c.length
-        c.append(key_states.contiguous(), value_states.contiguous())
+        key_states, value_states = key_states.contiguous(), value_states.contiguous()
+        if n > 1:
+            views = c.append_with_view(key_states, value_states, self.v_open)
+            if views is not None:
+                return views
+        c.append(key_states, value_states)
         # fp16 V tokens of the (new) open group, for fp16_view()
         open0 = c.length // g * g
         lo = max(open0, start)
@@ -221,6 +226,9 @@ class KIVILayer(CacheLayerMixin):
         dequantised full groups (fp32 code * scale -> fp16) and the fp16
         tokens of the open group."""
         c, g = self.cache, self.group_size
+        views = c.view(self.v_open)
+        if views is not None:
+            return views
         full = c.length // g * g
         k_q = _unpack_int4(c.k_q[:, :, :full])
         v_q = _unpack_int4(c.v_q[:, :, :full])

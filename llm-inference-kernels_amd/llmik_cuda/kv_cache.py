@@ -25,7 +25,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import (decode_attention_int4, decode_attention_int8, kivi_append_token_int4,
+from . import (_C, decode_attention_int4, decode_attention_int8, kivi_append_token_int4,
                quantize_k_per_channel_groupwise_int4_into, quantize_per_token_into,
                quantize_v_per_token_int4_into)
 
@@ -126,6 +126,10 @@ class Int4KIVICache:
                                    self.length, g)
             self.length += 1
             return
+        if _C.kivi_append_int4(k, v, self.k_open, None, self.k_q, self.k_scale, self.v_q, self.v_scale,
+                               self.length, g) is not None:
+            self.length += n
+            return
         quantize_v_per_token_int4_into(v, self.v_q, self.v_scale, self.length)
         pos = 0
         r = self.length % g
@@ -149,6 +153,26 @@ class Int4KIVICache:
             quantize_k_per_channel_groupwise_int4_into(
                 self.k_open[:, :, :rest], self.k_q, self.k_scale, self.length + pos, g)
         self.length += n
+
+    def append_with_view(self, k: torch.Tensor, v: torch.Tensor, v_open: torch.Tensor
+                         ) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """append(k, v), and the cache's fp16 view from the same launch: K and
+        V [batch, n_kv_heads, length, head_dim], fp16 code * scale of the full
+        groups and the fp16 tokens of the open one. v_open [batch,
+        n_kv_heads, group_size, head_dim] holds the open group's fp16 V tokens,
+        as k_open does K's, and is kept up to date. None, with nothing done,
+        where the launch does not take the call."""
+        n = _check_append(k, v, self.batch, self.n_kv_heads, self.head_dim, self.length, self.max_len)
+        views = _C.kivi_append_int4(k, v, self.k_open, v_open, self.k_q, self.k_scale, self.v_q, self.v_scale,
+                                    self.length, self.group_size)
+        if views is not None:
+            self.length += n
+        return views
+
+    def view(self, v_open: torch.Tensor) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """The fp16 view alone (see append_with_view)."""
+        return _C.kivi_append_int4(None, None, self.k_open, v_open, self.k_q, self.k_scale, self.v_q, self.v_scale,
+                                   self.length, self.group_size)
 
     def get_quantized_for_attention(self) -> Tuple[torch.Tensor, ...]:
         """(k_q, k_scale, v_q, v_scale, length): the whole buffers and the
