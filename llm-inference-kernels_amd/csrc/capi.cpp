@@ -94,10 +94,11 @@ LLMIK_API size_t llmik_attention_workspace_size(int batch, int n_heads, int n_kv
     if (batch <= 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim != 128 ||
         n_heads % n_kv_heads != 0 || seqlen <= 0)
         return 0;
-    // The size does not name the cache format: enough for the matrix-core
-    // kernels' plan and for the VALU kernel's.
-    const size_t mfma = plan_attention(batch, n_heads, n_kv_heads, seqlen, true).workspace_bytes;
-    const size_t valu = plan_attention(batch, n_heads, n_kv_heads, seqlen, false).workspace_bytes;
+    // The size does not name the cache format: enough for every kernel's plan.
+    // The INT8 and INT4 plans never split more often than the fp16 one.
+    const int cus = device_cu_count();
+    const size_t mfma = plan_attention(batch, n_heads, n_kv_heads, seqlen, AttnKind::F16, cus).workspace_bytes;
+    const size_t valu = plan_attention(batch, n_heads, n_kv_heads, seqlen, AttnKind::Valu, cus).workspace_bytes;
     return mfma > valu ? mfma : valu;
 }
 

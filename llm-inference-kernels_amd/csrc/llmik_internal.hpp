@@ -39,8 +39,9 @@ struct AttnPlan {
     size_t off_ml, off_o;
 };
 
-// mfma: the plan of the matrix-core kernels, else of the VALU kernel.
-AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, bool mfma);
+// Which kernels a plan is for: the matrix-core ones per cache format, or the VALU one.
+enum class AttnKind { F16, I8, I4, Valu };
+AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, AttnKind kind, int cus);
 // fp16 tile size knob (see llmik_attention_set_plan_override).
 void set_attention_plan_override(int f16_half_tiles);
 // W4A16 plan knobs (see llmik_w4a16_set_plan_override).

@@ -3,7 +3,8 @@ of them empty, or need several chunks per KV head.
 
 The plan takes up to 8 query heads of a KV head into one workgroup (4 where
 even one step per wave leaves CUs idle) and rounds 3 up to 4 and 5, 6 and 7 up
-to 8; more than 8 run in chunks whose last may be shorter. Every head's output
+to 8; more than 8 run in chunks whose last may be shorter. Slab counts that do
+not divide the CUs take plans of their own. Every head's output
 is compared with the oracle on the (dequantised) cache, max-abs <= 2e-3 as in
 the other attention tests, a repeated call returns the same bits, and values
 next to the output stay untouched.
@@ -47,6 +48,18 @@ CASES = [
     ("int4", 8, 8, 6, 1500, -1, 32),
     ("int4", 12, 4, 12, 900, 899, 64),   # two chunks of 6
     ("int4", 2, 8, 3, 400, -1, 32),
+    # slab counts that do not divide 256 CUs
+    ("fp16", 12, 8, 4, 1111, 1100, 0),   # 2 splits of 8 waves instead of 3
+    ("fp16", 17, 8, 4, 1281, -1, 0),     # 136 slabs: 3 splits of 4 waves
+    ("fp16", 17, 8, 4, 1279, 1279, 0),   # unsplit
+    ("fp16", 26, 8, 2, 700, 699, 0),     # 208 slabs, unsplit, 4 waves
+    ("fp16", 34, 8, 1, 515, 513, 0),     # 272 slabs in 3 splits
+    ("int8", 21, 8, 4, 1300, -1, 0),     # 168 slabs: 3 x 4 waves
+    ("int8", 32, 8, 1, 700, 697, 0),     # 256 slabs: 8 waves
+    ("int4", 21, 8, 4, 1300, 1299, 32),
+    ("int4", 24, 8, 4, 600, -1, 128),    # 192 slabs: 8 waves
+    ("int4", 33, 8, 1, 4100, 4097, 128),   # 264 slabs in 3 splits
+    ("int4", 32, 8, 1, 2561, -1, 64),    # 256 slabs: 8 waves
     ("int4", 4, 8, 8, 500, -1, 48),      # VALU kernel: chunks of 4
     ("int4", 4, 4, 7, 500, 499, 16),     # VALU kernel: one head per workgroup
 ]
