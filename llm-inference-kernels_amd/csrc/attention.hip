@@ -1315,9 +1315,24 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, Attn
     // INT8 B=32 S=3000 37.8, 32.3, S=500 8.9, 8.1; INT4 B=24 S=1500 13.1,
     // 12.2, B=27 S=200 5.4, 6.0, and with every CU filled B=32 S=3000 23.3,
     // 20.9, S=2048 16.2, 16.7.
+    // Short walks are not split at all: the hand-off (partials, counter,
+    // combine: three memory round trips) costs more than one or two further
+    // tiles per wave. us, split -> unsplit, B=1 / B=4 / B=12 (Hkv=8): fp16
+    // S=192 5.3 / 5.5 / 5.7 -> 4.65 / 5.1 / 5.2, S=224 5.3 / 5.4 / 5.8 -> 4.9 /
+    // 5.4 / 5.6, S=256 5.6 / 5.7 / 6.1 -> 5.1 / 5.85 / 6.3; INT8 S=256 5.45 /
+    // 5.55 / 5.85 -> 4.7 / 4.9 / 5.1, S=384 5.5 / 5.8 / 6.6 -> 5.3 / 5.7 / 5.8,
+    // S=448 5.5 / 6.0 / 7.1 -> 5.9 / 6.3 / 6.4; INT4 (4 waves) S=256 5.9 / 6.1
+    // / 6.3 -> 5.1 / 5.3 / 5.4, (8 waves) S=320 5.9 / 6.2 / 7.3 -> 6.0 / 6.2 /
+    // 6.3, S=384 6.0 / 6.2 / 7.7 -> 6.3 / 6.55 / 6.6.
+    const int short_walk = kind == AttnKind::F16 ? 224 : kind == AttnKind::I8 || base_wgs >= 48 ? 384 : 256;
+    const bool unsplit = mfma && few && seqlen > 4 * kTile && seqlen <= short_walk;
+    if (unsplit) {
+        want = 1;
+        pl.waves = kind == AttnKind::I4 && seqlen <= 256 ? 4 : 8;
+    }
     const long slot_cap = kMaxScratchSlots / pl.hpw / base_wgs;
     const bool short_ints = kind != AttnKind::F16 && seqlen < 4096;
-    if (mfma && !thin && !short_seq && base_wgs <= target) {
+    if (mfma && !unsplit && !thin && !short_seq && base_wgs <= target) {
         if (want * base_wgs > target) want = target / base_wgs;
         if (want == 1 && 3 * base_wgs <= 2 * target && seqlen >= 1280) {
             want = 3;

@@ -60,6 +60,15 @@ CASES = [
     ("int4", 24, 8, 4, 600, -1, 128),    # 192 slabs: 8 waves
     ("int4", 33, 8, 1, 4100, 4097, 128),   # 264 slabs in 3 splits
     ("int4", 32, 8, 1, 2561, -1, 64),    # 256 slabs: 8 waves
+    # short walks, unsplit
+    ("fp16", 2, 8, 4, 300, 129, 0),
+    ("fp16", 3, 8, 4, 224, -1, 0),
+    ("fp16", 3, 8, 4, 225, -1, 0),       # the first that is split
+    ("int8", 2, 8, 4, 384, 383, 0),
+    ("int8", 2, 8, 4, 385, -1, 0),
+    ("int4", 2, 8, 4, 256, 253, 32),
+    ("int4", 2, 8, 4, 257, -1, 32),
+    ("int4", 7, 8, 4, 384, 381, 64),
     ("int4", 4, 8, 8, 500, -1, 48),      # VALU kernel: chunks of 4
     ("int4", 4, 4, 7, 500, 499, 16),     # VALU kernel: one head per workgroup
 ]
