@@ -16,6 +16,7 @@
 // kernels/quant/quant_matmul.cu:586-597).
 #include <atomic>
 #include <cstdlib>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "llmik_internal.hpp"
@@ -1650,8 +1651,9 @@ __global__ __launch_bounds__(kG32Threads) void w4a16_gemm_mfma32_kernel(GemmPara
 }
 
 // ---------------------------------------------------------------------------
-// M >= 256 on 32x32x16 matrix cores (plan kind 7; N % 128 == 0, K % 64 == 0,
-// group size a power of two >= 32).
+// M >= 256 on 32x32x16 matrix cores (plan kind 7; N % 128 == 0, K % 64 == 0)
+// with scale groups of 256 and more, whose ends fall on any stage; groups of 32
+// to 128 run w4a16_gemm_reg_kernel below.
 //
 // A workgroup of 8 waves computes a tile of 256 rows by 128 columns over one
 // K split, in stages of 64 K, with both operands in LDS as fp16 rows of 128
@@ -1711,25 +1713,11 @@ __device__ __forceinline__ u32x4 i4x8_to_f16_natural(uint32_t w, uint32_t m, uin
     return out;
 }
 
-struct L7Words {
-    uint32_t w[2];      // packed rows (t >> 7) + 4 j of column t & 127
-    uint16_t s[2][2];   // [cb][u]: scales of the groups of chunks 1 and 3
+// The tile, K split and split-tile rank of a workgroup of the 256 x 128 GEMMs.
+struct L7Place {
+    int mtile, tile, split, nsplit, q;
 };
-
-// G32: group size 32 (two group ends per stage, four scale loads per lane
-// per stage; otherwise one group end and two).
-template <bool G32>
-__global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p) {
-    constexpr int kLoads = 4 + 2 + (G32 ? 4 : 2);   // vector memory instructions per stage
-    // Three separate activation slots: the copies into one slot and the
-    // fragment reads of another are then known not to alias, so the reads
-    // do not wait for copies still in flight.
-    __shared__ __attribute__((aligned(16))) uint8_t s_a0[kL7TM * 128];   // 3 x 32 KiB
-    __shared__ __attribute__((aligned(16))) uint8_t s_a1[kL7TM * 128];
-    __shared__ __attribute__((aligned(16))) uint8_t s_a2[kL7TM * 128];
-    __shared__ __attribute__((aligned(16))) uint8_t s_b[2][kL7TN * 128];   // 32 KiB
-    __shared__ uint32_t s_last;
-
+__device__ __forceinline__ L7Place l7_place(const GemmParams& p, const int bx, const int nwg) {
     // Tiles are numbered m-tile fastest (tl = tile * m_tiles + mtile). The
     // first full_tiles workgroups (whole rounds of the CUs) compute tiles
     // 0 .. full_tiles - 1 over all of K, XCD-contiguously when that count is
@@ -1741,7 +1729,6 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
     // neighbours on one XCD). A split tile q (its rank among the split
     // tiles) owns counter q and partial slots q * splits .. + splits - 1.
     const int F = p.full_tiles;
-    const int bx = blockIdx.x;
     // Unsplit tiles in groups of G m-tiles: index b -> (m-tile group, column
     // tile, m-tile in the group), so that consecutive indices (one XCD's
     // concurrent workgroups) cover G m-tiles of many column tiles.
@@ -1761,7 +1748,6 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
         q = 0;
     } else if (F == 0) {
         int b = bx;
-        const int nwg = gridDim.x;
         if ((nwg & 7) == 0) b = (b & 7) * (nwg >> 3) + (b >> 3);
         if (p.splits == 1) {
             tile_of(b, mtile, tile);
@@ -1781,6 +1767,27 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
         tile_of(F + q, mtile, tile);
         nsplit = p.splits;
     }
+    return {mtile, tile, split, nsplit, q};
+}
+
+struct L7Words {
+    uint32_t w[2];      // packed rows (t >> 7) + 4 j of column t & 127
+    uint16_t s[2];      // [cb]: scales of the stage's group
+};
+
+__global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p) {
+    constexpr int kLoads = 4 + 2 + 2;   // vector memory instructions per stage
+    // Three separate activation slots: the copies into one slot and the
+    // fragment reads of another are then known not to alias, so the reads
+    // do not wait for copies still in flight.
+    __shared__ __attribute__((aligned(16))) uint8_t s_a0[kL7TM * 128];   // 3 x 32 KiB
+    __shared__ __attribute__((aligned(16))) uint8_t s_a1[kL7TM * 128];
+    __shared__ __attribute__((aligned(16))) uint8_t s_a2[kL7TM * 128];
+    __shared__ __attribute__((aligned(16))) uint8_t s_b[2][kL7TN * 128];   // 32 KiB
+    __shared__ uint32_t s_last;
+
+    const L7Place pl = l7_place(p, blockIdx.x, gridDim.x);
+    const int mtile = pl.mtile, tile = pl.tile, split = pl.split, nsplit = pl.nsplit, q = pl.q;
 
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -1837,14 +1844,10 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
 #pragma unroll
         for (int j = 0; j < 2; ++j)
             g.w[j] = __builtin_amdgcn_raw_buffer_load_b32(rw, (int)(w_off + j * w_four), (int)(sc * w_stage), 0);
+        const uint32_t grp = (uint32_t)((4 * sc + 3) >> lcpg);
 #pragma unroll
-        for (int u = G32 ? 0 : 1; u < 2; ++u) {
-            const uint32_t grp = (uint32_t)((4 * sc + 1 + 2 * u) >> lcpg);
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb)
-                g.s[cb][u] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(s_off + 64u * cb),
-                                                                  (int)(grp * grp_bytes), 0);
-        }
+        for (int cb = 0; cb < 2; ++cb)
+            g.s[cb] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(s_off + 64u * cb), (int)(grp * grp_bytes), 0);
     };
     auto store_w = [&](const L7Words& g, int st) {
         uint8_t* slot = &s_b[(st - st0) & 1][0];
@@ -1869,9 +1872,9 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
     const int sw = c & 7;
 
     // One stage: chunk kk = 4 st + kc starts a scale group (or the split)
-    // only at even kc and ends one only at odd kc (groups are >= 2 chunks,
-    // splits whole stages); at kc = 1 only when the group is 32.
-    auto compute = [&](const uint8_t* sa, int st, const uint16_t (&scl)[2][2]) {
+    // only at kc = 0 and ends one only at kc = 3 (groups and splits are whole
+    // stages).
+    auto compute = [&](const uint8_t* sa, int st, const uint16_t (&scl)[2]) {
         const uint8_t* sb = &s_b[(st - st0) & 1][0];
         f16x8 aop[2][2], bop[2][2];   // [parity of kc][block]
         auto read_frags = [&](int kc) {
@@ -1891,7 +1894,7 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
             const int kk = 4 * st + kc;
             if (kc < 3) read_frags(kc + 1);
             const int x = kc & 1;
-            if ((kc & 1) == 0 && (((kk & cpg_mask) == 0) || kk == 4 * st0)) {
+            if (kc == 0 && (((kk & cpg_mask) == 0) || kk == 4 * st0)) {
 #pragma unroll
                 for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -1904,9 +1907,9 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
                     for (int cb = 0; cb < 2; ++cb)
                         cg[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop[x][rb], bop[x][cb], cg[rb][cb], 0, 0, 0);
             }
-            if ((kc == 3 || (G32 && kc == 1)) && (((kk & cpg_mask) == cpg_mask) || kk == 4 * st1 - 1)) {
-                const float s0 = h2f(scl[0][kc >> 1]);
-                const float s1 = h2f(scl[1][kc >> 1]);
+            if (kc == 3 && (((kk & cpg_mask) == cpg_mask) || kk == 4 * st1 - 1)) {
+                const float s0 = h2f(scl[0]);
+                const float s1 = h2f(scl[1]);
 #pragma unroll
                 for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -2059,6 +2062,322 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
 #pragma unroll
             for (int r = 0; r < 16; ++r) store_res(rb, cb, r, tot[rb][cb][r]);
     if (t == 0) p.counters[q] = 0u;
+}
+
+// ---------------------------------------------------------------------------
+// The same calls with scale groups of 32, 64 or 128: 128 x 128 tiles, the
+// weights dequantised into registers (plan kind 7; each 256 x 128 tile of the
+// plan is two workgroups).
+//
+// In the kernel above every MFMA operand comes from LDS: a wave's 64 x 64
+// block reads 4 KiB for 4 MFMAs of 16 K, 128 KiB of reads and 48 of writes per
+// 64-K stage at 128 bytes a cycle, 1408 LDS cycles for 1024 matrix cycles. Here
+// only the activations do. A workgroup of 4 waves (2 x 2 blocks of 64 x 64)
+// keeps 4 x 4 accumulators of v_mfma_f32_16x16x32_f16 per wave; lane (g, c)
+// loads the packed words of columns 4c .. 4c + 3, rows g and 4 + g of the
+// stage's 8, as two 16-byte loads two stages ahead, and each word becomes the
+// B operand of its column's block in registers (i4x8_to_f16_natural), so a
+// weight word is dequantised in 2 waves instead of once for 256 rows, but LDS
+// reads per MFMA fall to a quarter of a fragment (62 % of the matrix time).
+// Activations are copied straight into a ring of four 16-KiB slots, two stages
+// ahead; one bare barrier per stage. At 232 registers and 64 KiB of LDS two
+// workgroups share a CU, out of step, so that one's dequantisation and
+// barriers run beside the other's MFMAs. Products accumulate per scale group
+// from a zero C operand and are scaled at its end in fp32, as above (same
+// error against 64 bits: f32 output 1.0e-7 at K = 4096, 1.9e-7 at 14336).
+// us, kernel above -> this (M, K, N, group): 2048, 4096, 14336, 128: 260 -> 233
+// (1.03 PFLOP/s; a large fp16 library product reaches 1.31 on this card);
+// 2048, 14336, 4096: 249 -> 224; 2048, 4096, 4096: 74.3 -> 67.9; 512, 4096,
+// 14336: 70.8 -> 63.0; 256, 4096, 14336: 44.8 -> 37.7; 768, 14336, 4096: 122 ->
+// 103; 600, 11008, 4096: 96.4 -> 78.5; 4096, 4096, 14336: 506 -> 452; group 64,
+// 1000, 4096, 11008: 120 -> 109; group 32, 300, 4096, 14336: 90.7 -> 71.5.
+// Not kept: 256 x 128 tiles of 4 waves (128 x 64 blocks in 16-row strips, the
+// group scaling every 64 K instead of 128 for want of registers): 215 at the
+// first shape, but 1.4 times the fp32 error, and slower below two tiles per CU
+// (512, 4096, 14336: 74).
+// ---------------------------------------------------------------------------
+constexpr int kR8Threads = 256;
+constexpr int kR8TM = 128;
+
+template <int GROUP>   // 32, 64 or 128
+__global__ __launch_bounds__(kR8Threads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void w4a16_gemm_reg_kernel(GemmParams p) {
+    constexpr bool G32 = GROUP == 32;
+    constexpr int kLoads = 4 + 2 + (G32 ? 2 : 1);   // vector memory instructions per stage
+    // Four separate activation slots (see w4a16_gemm_lds_kernel).
+    __shared__ __attribute__((aligned(16))) uint8_t s_a0[kR8TM * 128];   // 4 x 16 KiB
+    __shared__ __attribute__((aligned(16))) uint8_t s_a1[kR8TM * 128];
+    __shared__ __attribute__((aligned(16))) uint8_t s_a2[kR8TM * 128];
+    __shared__ __attribute__((aligned(16))) uint8_t s_a3[kR8TM * 128];
+    __shared__ uint32_t s_last;
+
+    // Two workgroups per 256 x 128 tile of the plan, one per half of its rows,
+    // neighbours on one XCD (ids are dealt to the 8 XCDs round robin).
+    const int nplan = gridDim.x >> 1;
+    const int whole = nplan & ~7;
+    int bx, half;
+    if ((int)blockIdx.x < 2 * whole) {
+        const int i = blockIdx.x >> 3;
+        half = i & 1;
+        bx = ((i >> 1) << 3) | (blockIdx.x & 7);
+    } else {
+        const int r = blockIdx.x - 2 * whole;
+        half = r & 1;
+        bx = whole + (r >> 1);
+    }
+    const L7Place pl = l7_place(p, bx, nplan);
+    const int m0 = pl.mtile * kL7TM + half * kR8TM;
+    if (m0 >= p.M) return;   // the tile's second half may lie past the rows
+
+    const int t = threadIdx.x;
+    const int lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave & 1;
+    const int wn = wave >> 1;
+    const int c = lane & 15;
+    const int g = lane >> 4;
+
+    const int stages = p.K / 64;
+    const int st0 = pl.nsplit == 1 ? 0 : pl.split * p.wave_steps;
+    const int st1 = pl.nsplit == 1 ? stages : min(st0 + p.wave_steps, stages);
+    const int n0 = pl.tile * kL7TN + 64 * wn + 4 * c;   // this lane's four columns
+
+    const __amdgpu_buffer_rsrc_t rw = make_buffer_rsrc(p.w, (uint32_t)(p.K / 8) * p.N * 4u);
+    const __amdgpu_buffer_rsrc_t ra = make_buffer_rsrc(p.act, (uint32_t)p.M * p.K * 2u);
+    const __amdgpu_buffer_rsrc_t rs = make_buffer_rsrc(p.scale, (uint32_t)(p.K / p.group_size) * p.N * 2u);
+    // Activation copy: instruction i of wave w fills rows 8 (w + 4 i) .. + 7;
+    // lane l writes slot l % 8 of row 8 (w + 4 i) + l / 8, i.e. chunk
+    // (l % 8) ^ (l / 8) of that row. Rows past M point beyond the bound.
+    uint32_t a_off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = m0 + 8 * (wave + 4 * i) + (lane >> 3);
+        a_off[i] = (row < p.M) ? ((uint32_t)row * p.K * 2u + 16u * (uint32_t)((lane & 7) ^ (lane >> 3)))
+                               : 0x80000000u;
+    }
+    const uint32_t w_off = ((uint32_t)g * p.N + n0) * 4u;
+    const uint32_t w_half = (uint32_t)p.N * 16u;   // 4 packed rows
+    const uint32_t s_off = (uint32_t)n0 * 2u;
+    const uint32_t km = vgpr_const(0x00F0000Fu);
+    const uint32_t kx = vgpr_const(0x54806408u);
+
+    // Loads for stage st (clamped into the split: a stage past it re-reads the
+    // last one, in bounds, and is never used), always issued in full so that
+    // every stage issues the same number of vector memory instructions.
+    struct Words {
+        u32x4 w[2];              // rows g and 4 + g of the stage's 8, columns n0 .. + 3
+        u32x2 s[G32 ? 2 : 1];    // the columns' scales (group 32: per 32-K chunk)
+    };
+    auto load_a = [&](uint8_t* slot, int st) {
+        const uint32_t sc = (uint32_t)min(st, st1 - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                ra, (__attribute__((address_space(3))) void*)(slot + 1024 * (wave + 4 * i)), 16, (int)a_off[i],
+                (int)(sc * 128u), 0, 0);
+    };
+    auto load_w = [&](Words& d, int st) {
+        const int sc = min(st, st1 - 1);
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch)
+            d.w[ch] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(w_off + ch * w_half), (int)(sc * 2u * w_half), 0);
+#pragma unroll
+        for (int u = 0; u < (G32 ? 2 : 1); ++u) {
+            const uint32_t grp = G32 ? 2u * sc + u : (uint32_t)sc * 64u / GROUP;
+            d.s[u] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                rs, (int)s_off, (int)(grp * (uint32_t)p.N * 2u), 0));
+        }
+    };
+
+    f32x4 acc[4][4], cg[4][4];   // [16-row strip][column n0 + nb]
+    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            acc[i][nb] = zero4;
+            cg[i][nb] = zero4;
+        }
+    const int row0 = 64 * wm + c;
+    const int sw7 = c & 7;
+
+    // FIRST / LAST: the stage begins / ends a scale group (groups of 32 do both
+    // in every 32-K chunk). Known when compiled: a test at run time left copies
+    // of the accumulators around its branches and spilled.
+    auto stage = [&](const uint8_t* cur, uint8_t* far, Words& wd, int st, auto first, auto last) {
+        // Every load but the previous stage's kLoads is complete, so this
+        // wave's part of stage st's activations is in LDS; then the others'.
+        // (A bare barrier: __syncthreads would also wait for the copies in
+        // flight.) Slot `far` was last read two stages ago.
+        __builtin_amdgcn_s_waitcnt(kLoads | 0x0F70);
+        asm volatile("s_barrier" ::: "memory");
+        load_a(far, st + 2);
+        f16x8 b[2][4];
+        float sc[G32 ? 2 : 1][4];
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+                b[ch][nb] = __builtin_bit_cast(f16x8, i4x8_to_f16_natural(wd.w[ch][nb], km, kx));
+#pragma unroll
+        for (int u = 0; u < (G32 ? 2 : 1); ++u) {
+            const uint32_t s01 = wd.s[u][0], s23 = wd.s[u][1];
+            const f16x2 h01 = as_f16x2(s01), h23 = as_f16x2(s23);
+            sc[u][0] = (float)h01[0];
+            sc[u][1] = (float)h01[1];
+            sc[u][2] = (float)h23[0];
+            sc[u][3] = (float)h23[1];
+        }
+        load_w(wd, st + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+            f16x8 a[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                a[i] = __builtin_bit_cast(
+                    f16x8, *reinterpret_cast<const u32x4*>(cur + (row0 + 16 * i) * 128 + 16 * ((4 * ch + g) ^ sw7)));
+            if (G32 || (ch == 0 && decltype(first)::value)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb)
+                        cg[i][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[ch][nb], zero4, 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb)
+                        cg[i][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[ch][nb], cg[i][nb], 0, 0, 0);
+            }
+            if (G32 || (ch == 1 && decltype(last)::value)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            acc[i][nb][r] = fmaf(sc[G32 ? ch : 0][nb], cg[i][nb][r], acc[i][nb][r]);
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    Words w0, w1;
+    load_a(s_a0, st0);
+    load_w(w0, st0);
+    load_a(s_a1, st0 + 1);
+    load_w(w1, st0 + 1);
+    // Whole turns of the four slots, then the rest (a loop with an exit in the
+    // middle spills). Groups of 128 are two stages; the plan's splits begin and
+    // end on group boundaries.
+    constexpr std::integral_constant<bool, true> yes{};
+    constexpr std::integral_constant<bool, GROUP != 128> each{};
+    int st = st0;
+    for (; st + 3 < st1; st += 4) {
+        stage(s_a0, s_a2, w0, st, yes, each);
+        stage(s_a1, s_a3, w1, st + 1, each, yes);
+        stage(s_a2, s_a0, w0, st + 2, yes, each);
+        stage(s_a3, s_a1, w1, st + 3, each, yes);
+    }
+    if constexpr (GROUP == 128) {
+        if (st < st1) {
+            stage(s_a0, s_a2, w0, st, yes, each);
+            stage(s_a1, s_a3, w1, st + 1, each, yes);
+        }
+    } else {
+        if (st < st1) stage(s_a0, s_a2, w0, st, yes, yes);
+        if (st + 1 < st1) stage(s_a1, s_a3, w1, st + 1, yes, yes);
+        if (st + 2 < st1) stage(s_a2, s_a0, w0, st + 2, yes, yes);
+    }
+    __builtin_amdgcn_s_waitcnt(0);   // no copy into LDS outlives the workgroup
+
+    // D layout of v_mfma_f32_16x16x32: value r of lane (g, c) is row 4 g + r of
+    // the strip; block nb is column 4 c + nb of the wave's 64. Accesses are
+    // bounded by M rows: stores to rows past M are dropped.
+    const uint32_t esz = p.f32_out ? 4u : 2u;
+    const __amdgpu_buffer_rsrc_t ro = make_buffer_rsrc(p.out, (uint32_t)p.M * p.N * esz);   // plan: M N 4 < 2^31
+    const uint32_t e0 = (uint32_t)(m0 + 64 * wm + 4 * g) * p.N + n0;
+    auto store_row = [&](int i, int r, float v0, float v1, float v2, float v3) {
+        const uint32_t e = e0 + (uint32_t)(16 * i + r) * p.N;
+        if (p.f32_out)
+            __builtin_amdgcn_raw_buffer_store_b128(
+                make_u32x4(__float_as_uint(v0), __float_as_uint(v1), __float_as_uint(v2), __float_as_uint(v3)), ro,
+                (int)(e * 4u), 0, 0);
+        else
+            __builtin_amdgcn_raw_buffer_store_b64(
+                u32x2{(uint32_t)f2h_bits(v0) | ((uint32_t)f2h_bits(v1) << 16),
+                      (uint32_t)f2h_bits(v2) | ((uint32_t)f2h_bits(v3) << 16)}, ro, (int)(e * 2u), 0, 0);
+    };
+    if (pl.nsplit == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) store_row(i, r, acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]);
+        return;
+    }
+    // Split partials in the threads' own layout: block (i, nb) of thread t at
+    // float offset 4 (256 (4 i + nb) + t) of the half tile's slot. Counter
+    // 2 q + half.
+    constexpr uint32_t kHalfElems = kR8TM * kL7TN;
+    auto part_rsrc = [&](int sp) {
+        return make_buffer_rsrc(p.part + (2 * ((long)pl.q * pl.nsplit + sp) + half) * kHalfElems, kHalfElems * 4u);
+    };
+    auto blk_off = [&](int i, int nb) { return (uint32_t)((4 * i + nb) * kR8Threads + t) * 16u; };
+    uint32_t* const counter = &p.counters[2 * pl.q + half];
+    {
+        const __amdgpu_buffer_rsrc_t rp = part_rsrc(pl.split);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb)
+                publish_store16(rp, blk_off(i, nb),
+                                make_u32x4(__float_as_uint(acc[i][nb][0]), __float_as_uint(acc[i][nb][1]),
+                                           __float_as_uint(acc[i][nb][2]), __float_as_uint(acc[i][nb][3])));
+    }
+    publish_wait();
+    __syncthreads();
+    if (t == 0) s_last = arrive_last(counter, (uint32_t)pl.nsplit) ? 1u : 0u;
+    __syncthreads();
+    if (s_last == 0u) return;
+    // Last split of the half tile: the partials are added in split order (this
+    // workgroup's own from registers, the bits it stored), each split's 64
+    // values per thread loaded together.
+    f32x4 tot[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) tot[i][nb] = zero4;
+    for (int sp = 0; sp < pl.nsplit; ++sp) {
+        if (sp == pl.split) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) tot[i][nb] += acc[i][nb];
+            continue;
+        }
+        const __amdgpu_buffer_rsrc_t rp = part_rsrc(sp);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const u32x4 v = publish_load16(rp, blk_off(i, nb));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t bits = v[e];
+                    cg[i][nb][e] = __uint_as_float(bits);
+                }
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) tot[i][nb] += cg[i][nb];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) store_row(i, r, tot[i][0][r], tot[i][1][r], tot[i][2][r], tot[i][3][r]);
+    if (t == 0) *counter = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -2418,11 +2737,12 @@ static GemmPlan plan_w4a16_mode(int M, int N, int K, int group_size, int stream_
                 if (cost(sp) < best) { best = cost(sp); want = sp; }
             if (want == 1) full = 0, rest = tiles;   // no split: one plain launch order
         }
-        if (rest > kMaxCounters) want = 1, full = 0, rest = tiles;
+        if (2 * rest > kMaxCounters) want = 1, full = 0, rest = tiles;   // a counter per half tile
         if (want < 1) want = 1;
         if (want > stages) want = stages;
         int sps = (int)((stages + want - 1) / want);
         if (spg > 1 && sps > spg) sps = (sps + spg - 1) / spg * spg;
+        if (spg == 2 && sps == 1) sps = 2;   // w4a16_gemm_reg_kernel: groups of 128 are not cut
         pl.wave_steps = sps;
         pl.kp_per_split = 8 * sps;
         pl.splits = (stages + sps - 1) / sps;
@@ -2645,8 +2965,14 @@ int launch_w4a16(const void* act, const void* w, const void* scale, void* out, b
         p.m_tiles_ = pl.m_tiles;
         p.full_tiles = pl.full_tiles;
         const dim3 grid(pl.full_tiles + pl.split_tiles * pl.splits), blk(kL7Threads);
-        if (group_size == 32) hipLaunchKernelGGL(w4a16_gemm_lds_kernel<true>, grid, blk, 0, stream, p);
-        else hipLaunchKernelGGL(w4a16_gemm_lds_kernel<false>, grid, blk, 0, stream, p);
+        if (group_size <= 128) {
+            const dim3 g2(2 * grid.x), b2(kR8Threads);
+            if (group_size == 32) hipLaunchKernelGGL(w4a16_gemm_reg_kernel<32>, g2, b2, 0, stream, p);
+            else if (group_size == 64) hipLaunchKernelGGL(w4a16_gemm_reg_kernel<64>, g2, b2, 0, stream, p);
+            else hipLaunchKernelGGL(w4a16_gemm_reg_kernel<128>, g2, b2, 0, stream, p);
+        } else {
+            hipLaunchKernelGGL(w4a16_gemm_lds_kernel, grid, blk, 0, stream, p);
+        }
     } else if (pl.kind == 3) {
         const dim3 grid(pl.n_tiles * pl.splits * pl.m_tiles), blk(kMmaThreads);
         switch (pl.tile_m) {
