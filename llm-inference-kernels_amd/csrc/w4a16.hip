@@ -2556,9 +2556,6 @@ __global__ __launch_bounds__(256) void w4a16_dequantize_kernel(const uint32_t* _
 // llmik_w4a16_set_plan_override.
 constexpr long kStreamMinWeightBytes = 8L << 20;
 // Rows from which the 256 x 128 LDS-staged GEMM (kind 7) serves M > 16.
-#ifndef LLMIK_W4A16_LDS_MIN_M
-#define LLMIK_W4A16_LDS_MIN_M 256
-#endif
 
 namespace {
 int env_int(const char* name, bool as_flag) {
@@ -2691,10 +2688,20 @@ static GemmPlan plan_w4a16_mode(int M, int N, int K, int group_size, int stream_
             (pl.splits > 1) ? kCounterBytes + align_up((size_t)pl.splits * M * N * sizeof(float), 256) : 0;
         return pl;
     }
-    if (M >= LLMIK_W4A16_LDS_MIN_M && N % 128 == 0 && pow2_group && K % 64 == 0 &&
+    // From 129 rows kind 6's third 64-row tile starts a second round of the CUs
+    // wherever kind 7's rule holds ((K, N) = (4096, 14336), M=160 / 200: 45.5 /
+    // 45.6 against 35.7 / 37.4 us; (4096, 11008): 46.9 / 45.2 against 35.2).
+    // With 3 or 4 splits kind 7 pays only over a long K ((14336, 4096), M=300 /
+    // 400 / 512: 66.4 / 67.1 / 74.6 -> 55.8 / 62.3 / 66.4 in 4; at K = 4096,
+    // M=300, 23.9 against 25.1), and not at one 256-row tile (M=256, 42.0
+    // against 43.5). Groups of 256 and more (w4a16_gemm_lds_kernel): as before.
+    const bool reg_groups = group_size <= 128;
+    const long tiles7 = (long)((M + kL7TM - 1) / kL7TM) * (N / kL7TN);
+    if (M >= (reg_groups ? 129 : 256) && N % 128 == 0 && pow2_group && K % 64 == 0 &&
         (long)(K / 8) * N * 4 < (1L << 31) && (long)M * K * 2 < (1L << 31) &&
         (long)M * N * 4 < (1L << 31) &&
-        3L * ((M + kL7TM - 1) / kL7TM) * (N / kL7TN) > device_cu_count()) {
+        (3 * tiles7 > device_cu_count() ||
+         (reg_groups && M > 256 && K >= 8192 && 4 * tiles7 >= device_cu_count()))) {
         // 256 x 128 tiles with both operands staged in LDS; K splits (whole
         // scale groups where they allow) until the tiles fill the CUs once.
         // Chosen over kind 6 when its tiles need at most 2 splits (its split

@@ -1,4 +1,4 @@
-"""GPU parity: the 128 x 128-tile W4A16 GEMM of M >= 256 (groups 32, 64, 128) at
+"""GPU parity: the 128 x 128-tile W4A16 GEMM of M > 128 (groups 32, 64, 128) at
 the edges of its tiles, stages, groups and splits. Gate as in the other W4A16
 tests: the fp32 output within 2e-3 of the float64 product, the fp16 output its
 rounding bit for bit, a second call the same bits; values beside the output
@@ -27,6 +27,11 @@ CASES = [
     (300, 1152, 5760, 128),    # 90 tiles, 2 splits of 10 and 8 stages
     (770, 1024, 11008, 32),    # tiles past whole rounds split
     (1030, 512, 8192, 128),
+    (129, 256, 11008, 128),    # from 129 rows: one row tile, 2 splits of two stages
+    (255, 320, 11264, 64),
+    (160, 1088, 11008, 32),    # 17 stages in 2 splits
+    (300, 8192, 4096, 128),    # 64 tiles in 4 splits of 32 stages
+    (500, 8256, 4096, 64),     # 129 stages: 33, 33, 33 and 30
     (900, 4096, 4224, 64),     # an odd number of column tiles
 ]
 
