@@ -2708,7 +2708,7 @@ static GemmPlan plan_w4a16_mode(int M, int N, int K, int group_size, int stream_
         // hand-off is slower than kind 6's, and with 4 or more splits kind 6
         // is as fast or faster: M=512 (4096, 4096) 25.6 against 32.5 us,
         // (14336, 4096) 77.2 against 76.0; M=768, 2 splits, 46.8 -> 44.4 and
-        // 137.5 -> 126.4).
+        // 137.5 -> 126.4; w4a16_gemm_lds_kernel's figures).
         const int stages = K / 64;
         const int spg = group_size / 64;   // stages per scale group (0 when it is 32)
         pl.kind = 7;

@@ -277,12 +277,14 @@ _TARGET_LINEAR_NAMES = ("q_proj", "k_proj", "v_proj", "o_proj", "up_proj", "gate
 
 def dequant_path_threshold(N: int) -> int:
     """Rows from which dequantise + matmul (hipBLASLt) beats w4a16_gemm on
-    MI355X, measured at the Llama-3-8B shapes: w4a16_gemm is faster up to
-    1024 rows for N = 4096 (K = 4096 or 14336; 47.1 against 52.6 us and
-    129.1 against 151.5 at 1024, 70.2 against 64.1 at 1536) and up to 768
-    for N = 14336 (113.2 against 114.3; 139.3 against 122.6 at 1024). The
-    reference switches at 256
-    (integration/w4a16_patch.py:89), where w4a16_gemm is 2.0-2.4x faster.
+    MI355X, measured at the Llama-3-8B shapes with groups of 256 and more:
+    w4a16_gemm is faster up to 1024 rows for N = 4096 (K = 4096 or 14336;
+    47.1 against 52.6 us and 129.1 against 151.5 at 1024, 70.2 against 64.1
+    at 1536) and up to 768 for N = 14336 (113.2 against 114.3; 139.3 against
+    122.6 at 1024). Groups of 32 to 128 take 0.85-0.92 of those times (233 us
+    at 2048 rows of (4096, 14336), where dequantise + matmul takes 237), so
+    for them the two paths meet near 2048 rows. The reference switches at 256
+    (integration/w4a16_patch.py:89), where w4a16_gemm is 1.8-2.4x faster.
     Below the threshold the output is also the exact one (fp32 accumulation
     of unrounded weights, within 2e-3 of the float64 product; the fp16
     dequantised weights of the other path are not)."""
