@@ -2162,8 +2162,10 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
     const uint32_t kx = vgpr_const(0x54806408u);
 
     // Loads for stage st (clamped into the split: a stage past it re-reads the
-    // last one, in bounds, and is never used), always issued in full so that
-    // every stage issues the same number of vector memory instructions.
+    // last one, in bounds, and is never used). A stage issues its four copies
+    // before its register loads; of those the compiler merges a group of 128's
+    // second scale load with its first, and drops the ones for stages that the
+    // straight-line tail never reaches (see the waits below).
     struct Words {
         u32x4 w[2];              // rows g and 4 + g of the stage's 8, columns n0 .. + 3
         u32x2 s[G32 ? 2 : 1];    // the columns' scales (group 32: per 32-K chunk)
@@ -2204,12 +2206,16 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
     // FIRST / LAST: the stage begins / ends a scale group (groups of 32 do both
     // in every 32-K chunk). Known when compiled: a test at run time left copies
     // of the accumulators around its branches and spilled.
-    auto stage = [&](const uint8_t* cur, uint8_t* far, Words& wd, int st, auto first, auto last) {
-        // Every load but the previous stage's kLoads is complete, so this
-        // wave's part of stage st's activations is in LDS; then the others'.
+    auto stage = [&](const uint8_t* cur, uint8_t* far, Words& wd, int st, auto first, auto last, auto pending) {
+        // Every load but the newest `pending` is complete, so this wave's part
+        // of stage st's activations is in LDS; then the others'. After a
+        // stage with all its register loads that is kLoads; with its scale
+        // load merged, one register load of the stage before may be pending
+        // too, for which the compiler waits where it is used. After a stage of
+        // the tail, which may have issued its four copies alone, it is 4.
         // (A bare barrier: __syncthreads would also wait for the copies in
         // flight.) Slot `far` was last read two stages ago.
-        __builtin_amdgcn_s_waitcnt(kLoads | 0x0F70);
+        __builtin_amdgcn_s_waitcnt(decltype(pending)::value | 0x0F70);
         asm volatile("s_barrier" ::: "memory");
         load_a(far, st + 2);
         f16x8 b[2][4];
@@ -2265,30 +2271,33 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
     };
     Words w0, w1;
     load_a(s_a0, st0);
-    load_w(w0, st0);
     load_a(s_a1, st0 + 1);
+    __builtin_amdgcn_sched_barrier(0);   // the first stage's wait counts on this order
+    load_w(w0, st0);
     load_w(w1, st0 + 1);
     // Whole turns of the four slots, then the rest (a loop with an exit in the
     // middle spills). Groups of 128 are two stages; the plan's splits begin and
     // end on group boundaries.
     constexpr std::integral_constant<bool, true> yes{};
     constexpr std::integral_constant<bool, GROUP != 128> each{};
+    constexpr std::integral_constant<int, kLoads> full{};
+    constexpr std::integral_constant<int, 4> tail{};
     int st = st0;
     for (; st + 3 < st1; st += 4) {
-        stage(s_a0, s_a2, w0, st, yes, each);
-        stage(s_a1, s_a3, w1, st + 1, each, yes);
-        stage(s_a2, s_a0, w0, st + 2, yes, each);
-        stage(s_a3, s_a1, w1, st + 3, each, yes);
+        stage(s_a0, s_a2, w0, st, yes, each, full);
+        stage(s_a1, s_a3, w1, st + 1, each, yes, full);
+        stage(s_a2, s_a0, w0, st + 2, yes, each, full);
+        stage(s_a3, s_a1, w1, st + 3, each, yes, full);
     }
     if constexpr (GROUP == 128) {
         if (st < st1) {
-            stage(s_a0, s_a2, w0, st, yes, each);
-            stage(s_a1, s_a3, w1, st + 1, each, yes);
+            stage(s_a0, s_a2, w0, st, yes, each, full);
+            stage(s_a1, s_a3, w1, st + 1, each, yes, tail);
         }
     } else {
-        if (st < st1) stage(s_a0, s_a2, w0, st, yes, yes);
-        if (st + 1 < st1) stage(s_a1, s_a3, w1, st + 1, yes, yes);
-        if (st + 2 < st1) stage(s_a2, s_a0, w0, st + 2, yes, yes);
+        if (st < st1) stage(s_a0, s_a2, w0, st, yes, yes, full);
+        if (st + 1 < st1) stage(s_a1, s_a3, w1, st + 1, yes, yes, tail);
+        if (st + 2 < st1) stage(s_a2, s_a0, w0, st + 2, yes, yes, tail);
     }
     __builtin_amdgcn_s_waitcnt(0);   // no copy into LDS outlives the workgroup
 
@@ -2555,7 +2564,6 @@ __global__ __launch_bounds__(256) void w4a16_dequantize_kernel(const uint32_t* _
 // LLMIK_W4A16_STREAM_SPLITS when the library loads, and settable with
 // llmik_w4a16_set_plan_override.
 constexpr long kStreamMinWeightBytes = 8L << 20;
-// Rows from which the 256 x 128 LDS-staged GEMM (kind 7) serves M > 16.
 
 namespace {
 int env_int(const char* name, bool as_flag) {
