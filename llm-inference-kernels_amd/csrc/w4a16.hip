@@ -2103,7 +2103,6 @@ template <int GROUP>   // 32, 64 or 128
 __global__ __launch_bounds__(kR8Threads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void w4a16_gemm_reg_kernel(GemmParams p) {
     constexpr bool G32 = GROUP == 32;
-    constexpr int kLoads = 4 + 2 + (G32 ? 2 : 1);   // vector memory instructions per stage
     // Four separate activation slots (see w4a16_gemm_lds_kernel).
     __shared__ __attribute__((aligned(16))) uint8_t s_a0[kR8TM * 128];   // 4 x 16 KiB
     __shared__ __attribute__((aligned(16))) uint8_t s_a1[kR8TM * 128];
@@ -2162,10 +2161,8 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
     const uint32_t kx = vgpr_const(0x54806408u);
 
     // Loads for stage st (clamped into the split: a stage past it re-reads the
-    // last one, in bounds, and is never used). A stage issues its four copies
-    // before its register loads; of those the compiler merges a group of 128's
-    // second scale load with its first, and drops the ones for stages that the
-    // straight-line tail never reaches (see the waits below).
+    // last one, in bounds, and is never used): four copies, two loads of words
+    // and, where a group ends in the stage (LAST), its scales.
     struct Words {
         u32x4 w[2];              // rows g and 4 + g of the stage's 8, columns n0 .. + 3
         u32x2 s[G32 ? 2 : 1];    // the columns' scales (group 32: per 32-K chunk)
@@ -2183,8 +2180,11 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
 #pragma unroll
         for (int ch = 0; ch < 2; ++ch)
             d.w[ch] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(w_off + ch * w_half), (int)(sc * 2u * w_half), 0);
+    };
+    auto load_s = [&](Words& d, int st, auto last) {
+        const int sc = min(st, st1 - 1);
 #pragma unroll
-        for (int u = 0; u < (G32 ? 2 : 1); ++u) {
+        for (int u = 0; u < (decltype(last)::value ? (G32 ? 2 : 1) : 0); ++u) {
             const uint32_t grp = G32 ? 2u * sc + u : (uint32_t)sc * 64u / GROUP;
             d.s[u] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
                 rs, (int)s_off, (int)(grp * (uint32_t)p.N * 2u), 0));
@@ -2205,18 +2205,24 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
 
     // FIRST / LAST: the stage begins / ends a scale group (groups of 32 do both
     // in every 32-K chunk). Known when compiled: a test at run time left copies
-    // of the accumulators around its branches and spilled.
+    // of the accumulators around its branches and spilled. Stage st + 2, whose
+    // loads stage st issues, begins and ends groups as st does.
     auto stage = [&](const uint8_t* cur, uint8_t* far, Words& wd, int st, auto first, auto last, auto pending) {
-        // Every load but the newest `pending` is complete, so this wave's part
-        // of stage st's activations is in LDS; then the others'. After a
-        // stage with all its register loads that is kLoads; with its scale
-        // load merged, one register load of the stage before may be pending
-        // too, for which the compiler waits where it is used. After a stage of
-        // the tail, which may have issued its four copies alone, it is 4.
-        // (A bare barrier: __syncthreads would also wait for the copies in
-        // flight.) Slot `far` was last read two stages ago.
+        // Every load but the newest `pending` is complete. That many at least
+        // were issued by the stage before (a tail's, whose register loads the
+        // compiler drops where no stage is left to use them, issues its four
+        // copies), so all loads of the stages before that are, in whatever
+        // order a stage's loads were issued: this wave's part of stage st's
+        // activations is in LDS, then the others'. (A bare barrier:
+        // __syncthreads would also wait for the copies in flight.) Slot `far`
+        // was last read two stages ago.
         __builtin_amdgcn_s_waitcnt(decltype(pending)::value | 0x0F70);
         asm volatile("s_barrier" ::: "memory");
+        // The scales first: the stage that waits for all of this one's loads
+        // needs its words at once and its scales last.
+        Words cw = wd;
+        load_s(wd, st + 2, last);
+        __builtin_amdgcn_sched_barrier(0);
         load_a(far, st + 2);
         f16x8 b[2][4];
         float sc[G32 ? 2 : 1][4];
@@ -2224,10 +2230,10 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
         for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb)
-                b[ch][nb] = __builtin_bit_cast(f16x8, i4x8_to_f16_natural(wd.w[ch][nb], km, kx));
+                b[ch][nb] = __builtin_bit_cast(f16x8, i4x8_to_f16_natural(cw.w[ch][nb], km, kx));
 #pragma unroll
-        for (int u = 0; u < (G32 ? 2 : 1); ++u) {
-            const uint32_t s01 = wd.s[u][0], s23 = wd.s[u][1];
+        for (int u = 0; u < (decltype(last)::value ? (G32 ? 2 : 1) : 0); ++u) {
+            const uint32_t s01 = cw.s[u][0], s23 = cw.s[u][1];
             const f16x2 h01 = as_f16x2(s01), h23 = as_f16x2(s23);
             sc[u][0] = (float)h01[0];
             sc[u][1] = (float)h01[1];
@@ -2269,25 +2275,30 @@ void w4a16_gemm_reg_kernel(GemmParams p) {
         }
         __builtin_amdgcn_s_setprio(0);
     };
-    Words w0, w1;
-    load_a(s_a0, st0);
-    load_a(s_a1, st0 + 1);
-    __builtin_amdgcn_sched_barrier(0);   // the first stage's wait counts on this order
-    load_w(w0, st0);
-    load_w(w1, st0 + 1);
     // Whole turns of the four slots, then the rest (a loop with an exit in the
     // middle spills). Groups of 128 are two stages; the plan's splits begin and
     // end on group boundaries.
     constexpr std::integral_constant<bool, true> yes{};
     constexpr std::integral_constant<bool, GROUP != 128> each{};
-    constexpr std::integral_constant<int, kLoads> full{};
+    // Vector memory instructions of a stage that ends a group, of one that need
+    // not (groups of 128), and of one of the tail.
+    constexpr std::integral_constant<int, 4 + 2 + (G32 ? 2 : 1)> full{};
+    constexpr std::integral_constant<int, 4 + 2 + (G32 ? 2 : GROUP != 128 ? 1 : 0)> open{};
     constexpr std::integral_constant<int, 4> tail{};
+    Words w0{}, w1{};
+    load_s(w0, st0, each);
+    load_a(s_a0, st0);
+    load_w(w0, st0);
+    __builtin_amdgcn_sched_barrier(0);   // the first wait counts the second stage's loads
+    load_s(w1, st0 + 1, yes);
+    load_a(s_a1, st0 + 1);
+    load_w(w1, st0 + 1);
     int st = st0;
     for (; st + 3 < st1; st += 4) {
         stage(s_a0, s_a2, w0, st, yes, each, full);
-        stage(s_a1, s_a3, w1, st + 1, each, yes, full);
+        stage(s_a1, s_a3, w1, st + 1, each, yes, open);
         stage(s_a2, s_a0, w0, st + 2, yes, each, full);
-        stage(s_a3, s_a1, w1, st + 3, each, yes, full);
+        stage(s_a3, s_a1, w1, st + 3, each, yes, open);
     }
     if constexpr (GROUP == 128) {
         if (st < st1) {
