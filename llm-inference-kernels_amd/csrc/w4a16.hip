@@ -1894,6 +1894,12 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
             const int kk = 4 * st + kc;
             if (kc < 3) read_frags(kc + 1);
             const int x = kc & 1;
+            // The stage's second half is scheduled by itself: across the whole
+            // stage the compiler spread the fragment reads worse (us, without ->
+            // with, group 256: M=352 (4096, 11008) 70.6 -> 68.3, M=300 (4096,
+            // 14336) 69.7 -> 67.0, M=532 (2048, 8192) 38.3 -> 36.8, M=2048 (4096,
+            // 14336) 261 -> 258).
+            if (kc == 2) __builtin_amdgcn_sched_barrier(0);
             if (kc == 0 && (((kk & cpg_mask) == 0) || kk == 4 * st0)) {
 #pragma unroll
                 for (int rb = 0; rb < 2; ++rb)
