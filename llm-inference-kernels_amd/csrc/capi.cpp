@@ -4,6 +4,7 @@
 // kernels/common/cuda_utils.cuh:12-24) and forwards to the launchers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -95,11 +96,11 @@ LLMIK_API size_t llmik_attention_workspace_size(int batch, int n_heads, int n_kv
         n_heads % n_kv_heads != 0 || seqlen <= 0)
         return 0;
     // The size does not name the cache format: enough for every kernel's plan.
-    // The INT8 and INT4 plans never split more often than the fp16 one.
     const int cus = device_cu_count();
-    const size_t mfma = plan_attention(batch, n_heads, n_kv_heads, seqlen, AttnKind::F16, cus).workspace_bytes;
-    const size_t valu = plan_attention(batch, n_heads, n_kv_heads, seqlen, AttnKind::Valu, cus).workspace_bytes;
-    return mfma > valu ? mfma : valu;
+    size_t need = 0;
+    for (const AttnKind kind : {AttnKind::F16, AttnKind::I8, AttnKind::I4, AttnKind::Valu})
+        need = std::max(need, plan_attention(batch, n_heads, n_kv_heads, seqlen, kind, cus).workspace_bytes);
+    return need;
 }
 
 LLMIK_API llmik_status llmik_decode_attention_f16(const void* q, const void* k, const void* v,

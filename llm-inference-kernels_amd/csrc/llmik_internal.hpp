@@ -27,6 +27,13 @@ int check_launch();
 int device_cu_count();
 
 // ---- attention -------------------------------------------------------------
+constexpr int kHeadDim = 128;
+constexpr int kTile = 32;   // tokens per wave step of the MFMA kernel
+#ifndef LLMIK_ATTN_WGS_PER_CU
+#define LLMIK_ATTN_WGS_PER_CU 1
+#endif
+constexpr int kAttnWgsPerCu = LLMIK_ATTN_WGS_PER_CU;
+
 struct AttnPlan {
     int hpw;             // query heads a workgroup computes (1, 2, 4 or 8)
     int n_hchunks;       // head chunks per kv head
