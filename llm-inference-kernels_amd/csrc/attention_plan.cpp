@@ -9,19 +9,19 @@ namespace llmik {
 
 namespace {
 
-// Heads per workgroup. MFMA kernels: all query heads of a kv head together up
-// to `most` (4 or 8) of them, more in equal chunks; the 16 rows of a matrix
-// operand cost the same for 3 heads as for 4 and for 5 as for 8. VALU kernel,
-// whose work grows with every head: the power of two up to 4 that divides.
-void head_chunks(int gqa, bool mfma, int most, AttnPlan& pl) {
-    if (mfma) {
-        pl.n_hchunks = (gqa + most - 1) / most;
-        pl.heads_per_chunk = (gqa + pl.n_hchunks - 1) / pl.n_hchunks;
-        pl.hpw = pl.heads_per_chunk > 4 ? 8 : pl.heads_per_chunk > 2 ? 4 : pl.heads_per_chunk;
-        return;
-    }
-    pl.hpw = gqa % 4 == 0 ? 4 : gqa % 2 == 0 ? 2 : 1;
-    pl.heads_per_chunk = pl.hpw;
+// Heads per workgroup, two ways. All query heads of a kv head together up to
+// `most` (4 or 8) of them, more in equal chunks: the 16 rows of a matrix
+// operand cost the same for 3 heads as for 4 and for 5 as for 8.
+void joint_chunks(int gqa, int most, AttnPlan& pl) {
+    pl.n_hchunks = (gqa + most - 1) / most;
+    pl.heads_per_chunk = (gqa + pl.n_hchunks - 1) / pl.n_hchunks;
+    pl.hpw = pl.heads_per_chunk > 4 ? 8 : pl.heads_per_chunk > 2 ? 4 : pl.heads_per_chunk;
+}
+// The power of two up to 4 that divides them: the VALU kernel, whose work grows
+// with every head, and small INT4 calls.
+int dividing_heads(int gqa) { return gqa % 4 == 0 ? 4 : gqa % 2 == 0 ? 2 : 1; }
+void dividing_chunks(int gqa, AttnPlan& pl) {
+    pl.hpw = pl.heads_per_chunk = dividing_heads(gqa);
     pl.n_hchunks = gqa / pl.hpw;
 }
 
@@ -48,7 +48,25 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, Attn
     // even one step per wave would leave CUs idle, chunks of up to 4 heads
     // (twice the workgroups) finish sooner: INT4 H=64 B=2 S=2048 8.95 against
     // 8.35, INT8 B=1 S=2000 7.6 against 7.5.
-    head_chunks(gqa, mfma, (long)batch * n_kv_heads * ((gqa + 7) / 8) * splits8 < target ? 4 : 8, pl);
+    // INT4 calls whose dividing chunks, in steps of 8 waves (4 waves from 385
+    // to 512 tokens, as split below), find a CU each keep those, up to 5 of a kv
+    // head and 2048 tokens (longer walks are better off with fewer, longer
+    // splits, below): a workgroup does a few tiles only, and its time is the
+    // softmax and the merge of its own heads, not the cache, which the chunks
+    // read again. us, joint -> dividing, caches read in turn from HBM: H=24
+    // Hkv=8 (3 x 1) B=1 S=120 4.15 -> 3.81, S=400 5.83 -> 5.45, S=1145 7.17 ->
+    // 6.76, B=4 S=256 4.96 -> 4.72; H=48 Hkv=8 (3 x 2) B=1 S=2000 8.24 -> 7.66;
+    // H=40 Hkv=8 (5 x 1) B=1 S=400 5.96 -> 5.55. With more workgroups than CUs
+    // (H=24 B=3 S=400) 6.02 -> 6.34. Not 7 chunks (H=28 Hkv=4 B=4 S=120 4.35 ->
+    // 4.42, S=256 5.06 -> 5.27); fp16 and INT8 are even (B=4 S=120, H=24 Hkv=8:
+    // 4.28, 4.26 and 3.71, 3.81).
+    const long dividing = gqa / dividing_heads(gqa);
+    const long small_splits = seqlen > 384 && seqlen <= 512 ? (seqlen + 4 * kTile - 1) / (4 * kTile) : splits8;
+    if (!mfma || (kind == AttnKind::I4 && dividing <= 5 && splits8 <= 8 &&
+                  (long)batch * n_kv_heads * dividing * small_splits <= target))
+        dividing_chunks(gqa, pl);
+    else
+        joint_chunks(gqa, (long)batch * n_kv_heads * ((gqa + 7) / 8) * splits8 < target ? 4 : 8, pl);
     const long base_wgs = (long)batch * n_kv_heads * pl.n_hchunks;
     // Aim for kAttnWgsPerCu workgroups per CU. Calls that must split the
     // sequence to fill the chip use 8-wave workgroups (more loads in flight
@@ -129,6 +147,17 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, Attn
     }
     const int step = kTile * pl.waves;
     const long max_useful = (seqlen + step - 1) / step;
+    // INT4 heads that were joined leave fewer slabs for the same CUs, which
+    // would be cut into more splits of one tile per wave: above 10 of those,
+    // half as many of two tiles, as the combine's time grows with their
+    // number. us, caches from HBM, H=24 Hkv=8: B=1 S=2700 8.26 -> 8.05, S=4500
+    // 10.10 -> 8.94, S=7500 11.56 -> 9.59, B=2 S=3500 10.03 -> 8.92; H=28
+    // Hkv=4 B=1 S=5900 10.70 -> 9.22; H=40 Hkv=8 B=1 S=3500 10.00 -> 8.91. At 8
+    // splits it is even (B=1 S=2000 7.51, 7.50), with 4 slabs up to 4 % slower
+    // below 3500 tokens (H=12 Hkv=4 S=2700 7.71 -> 7.94).
+    if (kind == AttnKind::I4 && pl.n_hchunks < dividing && !unsplit && !thin && !short_seq && max_useful > 10 &&
+        want >= max_useful)
+        want = (max_useful + 1) / 2;
     if (want > max_useful) want = max_useful;
     if (want > kMaxAttnSplits) want = kMaxAttnSplits;
     if (base_wgs > kMaxCounters) want = 1;   // enough workgroups without splitting

@@ -101,3 +101,23 @@ def test_workspace_query_covers_every_format(plans):
                 need = lib.llmik_attention_workspace_size(b, h, hkv, s, 128)
                 most = max(_plan(plans, b, h, hkv, s, kind, cus)["workspace"] for kind in (F16, I8, I4, VALU))
                 assert need == most, (b, h, hkv, s)
+
+
+@pytest.mark.parametrize("b,h,hkv,s,kind,chunks", [
+    (1, 24, 8, 120, I4, 3), (8, 24, 8, 120, I4, 3), (11, 24, 8, 120, I4, 1),   # 264 workgroups: joint
+    (1, 48, 8, 1145, I4, 3), (2, 40, 8, 300, I4, 5), (1, 48, 8, 2048, I4, 3), (1, 48, 8, 2049, I4, 2),
+    (2, 24, 8, 400, I4, 3), (3, 24, 8, 400, I4, 1), (1, 28, 4, 120, I4, 2), (1, 24, 8, 120, F16, 1), (1, 24, 8, 120, I8, 1), (1, 24, 8, 120, VALU, 3),
+    (1, 64, 8, 300, I4, 2), (1, 32, 8, 300, I4, 1),
+])
+def test_small_int4_calls_keep_dividing_chunks(plans, b, h, hkv, s, kind, chunks):
+    assert _plan(plans, b, h, hkv, s, kind)["n_hchunks"] == chunks
+
+
+@pytest.mark.parametrize("b,h,hkv,s,kind,splits", [
+    (1, 24, 8, 2560, I4, 10), (1, 24, 8, 2561, I4, 6), (1, 24, 8, 5900, I4, 12), (2, 28, 4, 2700, I4, 6),
+    (1, 24, 8, 9000, I4, 18),                            # 32 wanted of 36: two tiles per wave already
+    (1, 32, 8, 5900, I4, 24),                            # heads that were not joined
+    (1, 24, 8, 5900, F16, 24), (1, 24, 8, 5900, I8, 24), (4, 32, 8, 5900, I4, 8),
+])
+def test_int4_splits_of_one_tile_per_wave(plans, b, h, hkv, s, kind, splits):
+    assert _plan(plans, b, h, hkv, s, kind)["n_splits"] == splits
