@@ -355,8 +355,9 @@ int64_t token_rows_or_zero(const Tensor& x) {
 // and, with v_open, the fp16 view of the whole cache: (k, v) views, or (None,
 // None) without v_open. k and v may be None (the view alone). Returns None
 // where the launch does not take the call (a head_dim other than 128, groups
-// above 128, rows that are not equally spaced or not 16-byte aligned): the
-// caller's general path then serves or refuses it. The cache tensors are the
+// above 128, rows that are not equally spaced or not 16-byte aligned, tensors
+// whose gradients are recorded): the caller's general path then serves or
+// refuses it. The cache tensors are the
 // cache object's own; its shapes are re-checked here because the kernel
 // trusts them.
 py::object kivi_append_int4(const std::optional<Tensor>& k, const std::optional<Tensor>& v, const Tensor& k_open,
@@ -393,6 +394,10 @@ py::object kivi_append_int4(const std::optional<Tensor>& k, const std::optional<
     }
     for (const Tensor& t : all)
         if (t.device() != k_q.device() || (uintptr_t)t.data_ptr() % 16 != 0) return py::none();
+    // The open group's tokens pass unchanged into k_open, v_open and the views:
+    // where autograd follows them, the general path records that.
+    for (const Tensor& t : all)
+        if ((at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined()) return py::none();
     if (length < 0 || length + n > max_len) return py::none();
     const c10::DeviceGuard guard(k_q.device());
     Tensor kv, vv;

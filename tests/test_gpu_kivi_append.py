@@ -135,6 +135,55 @@ def test_rows_the_launch_does_not_take(llmik, cuda):
         kvc.Int4KIVICache(2, 2, 64, 32, device=cuda).append(k, odd)
 
 
+def _layer_run(cuda, record):
+    """Two prefill chunks through a layer; the views and what autograd says of them."""
+    from llmik_cuda.hf import KIVILayer
+    layer = KIVILayer(128, 32)
+    ks, vs = [], []
+    for i, n in enumerate((45, 40)):   # 13 tokens open, then 21
+        ks.append(_tokens(cuda, 2, 2, n, 2 * i))
+        vs.append(_tokens(cuda, 2, 2, n, 2 * i + 1))
+    return layer, ks, vs, record(layer, ks, vs)
+
+
+def test_gradients_of_the_open_group(llmik, cuda):
+    """The views hold the open group's tokens themselves: their gradient is the
+    view's, the quantised tokens' is zero, as through the general path."""
+    def record(layer, ks, vs):
+        for t in ks + vs:
+            t.requires_grad_(True)
+        for k, v in zip(ks, vs):
+            view_k, view_v = layer.update(k, v)
+        assert view_k.requires_grad and view_v.requires_grad
+        w = torch.arange(1, 86, device=cuda, dtype=torch.float16)[:, None] / 64
+        ((view_k * w).sum() + 2 * (view_v * w).sum()).backward()
+        return w, layer.fp16_view()
+
+    layer, ks, vs, (w, later) = _layer_run(cuda, record)
+    for t, f in ((ks[1], 1), (vs[1], 2)):
+        want = torch.zeros_like(t)
+        want[:, :, -21:] = f * w[-21:]
+        assert torch.equal(t.grad, want)
+    assert all(t.grad is None or not t.grad.any() for t in (ks[0], vs[0]))
+    with torch.no_grad():
+        a, b = layer.fp16_view()
+    assert not a.requires_grad and torch.equal(a, later[0]) and torch.equal(b, later[1])
+
+
+def test_forward_mode_tangents_of_the_open_group(llmik, cuda):
+    import torch.autograd.forward_ad as fw
+
+    def record(layer, ks, vs):
+        with fw.dual_level():
+            for k, v in zip(ks, vs):
+                views = layer.update(fw.make_dual(k, torch.ones_like(k)), fw.make_dual(v, 2 * torch.ones_like(v)))
+            return [fw.unpack_dual(t).tangent for t in views]
+
+    *_, tangents = _layer_run(cuda, record)
+    for t, f in zip(tangents, (1, 2)):
+        assert bool((t[:, :, -21:] == f).all()) and not bool(t[:, :, :-21].any())
+
+
 def test_capture_and_replay(llmik, cuda):
     k, v = _tokens(cuda, 2, 4, 90, 1), _tokens(cuda, 2, 4, 90, 2)
     eager = kvc.Int4KIVICache(2, 4, 128, 32, device=cuda)
