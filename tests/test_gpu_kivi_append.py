@@ -17,6 +17,20 @@ def _general(monkeypatch):
     monkeypatch.setattr(kvc, "_C", types.SimpleNamespace(kivi_append_int4=lambda *a: None))
 
 
+@pytest.fixture
+def launches(monkeypatch):
+    """Whether the one-launch path took each call that the cache classes made of it."""
+    taken, real = [], kvc._C.kivi_append_int4
+
+    def count(*args):
+        out = real(*args)
+        taken.append(out is not None)
+        return out
+
+    monkeypatch.setattr(kvc, "_C", types.SimpleNamespace(kivi_append_int4=count))
+    return taken
+
+
 def _tokens(cuda, B, H, n, seed, special=False):
     g = torch.Generator(device=cuda).manual_seed(seed)
     x = torch.randn((B, H, n, 128), generator=g, device=cuda, dtype=torch.float16)
@@ -55,7 +69,7 @@ SEQUENCES = [
 
 @pytest.mark.parametrize("special", [False, True])
 @pytest.mark.parametrize("g,appends", SEQUENCES, ids=[f"g{s[0]}" for s in SEQUENCES])
-def test_appends_and_views_equal_the_general_path(llmik, cuda, monkeypatch, g, appends, special):
+def test_appends_and_views_equal_the_general_path(llmik, cuda, monkeypatch, launches, g, appends, special):
     from llmik_cuda.hf import KIVILayer
     B, H, max_len = 2, 3, sum(appends) + 5
 
@@ -74,6 +88,8 @@ def test_appends_and_views_equal_the_general_path(llmik, cuda, monkeypatch, g, a
         return layer, plain, views
 
     layer, plain, views = run()
+    # layer updates and plain appends of several tokens, and the other views
+    assert launches == [True] * (2 * len(appends) + sum(n > 1 for n in appends))
     _general(monkeypatch)
     layer0, plain0, views0 = run()
     for a, b in ((layer.cache, layer0.cache), (plain, plain0)):
@@ -89,7 +105,7 @@ def test_appends_and_views_equal_the_general_path(llmik, cuda, monkeypatch, g, a
 
 
 @pytest.mark.parametrize("g,n", [(128, 700), (100, 301), (64, 513), (33, 100)])
-def test_many_rows(llmik, cuda, monkeypatch, g, n):
+def test_many_rows(llmik, cuda, monkeypatch, launches, g, n):
     """More workgroups than CUs: the other workgroup size of groups above 64."""
     k, v = _tokens(cuda, 8, 9, n, 5), _tokens(cuda, 8, 9, n, 6)
     caches = []
@@ -99,24 +115,26 @@ def test_many_rows(llmik, cuda, monkeypatch, g, n):
         c = kvc.Int4KIVICache(8, 9, n + 1, g, device=cuda)
         c.append(k, v)
         caches.append(c)
+    assert launches == [True]
     a, b = caches
     for name in ("k_q", "k_scale", "v_q", "v_scale"):
         assert torch.equal(getattr(a, name), getattr(b, name)), name
     assert torch.equal(a.k_open[:, :, :n % g], b.k_open[:, :, :n % g])
 
 
-def test_nothing_past_the_live_length_is_written(llmik, cuda):
+def test_nothing_past_the_live_length_is_written(llmik, cuda, launches):
     cache = kvc.Int4KIVICache(2, 2, 200, 32, device=cuda)
     for t in (cache.k_q, cache.v_q):
         t.fill_(77)
     for t in (cache.k_scale, cache.v_scale):
         t.fill_(7.0)
     cache.append(_tokens(cuda, 2, 2, 70, 1), _tokens(cuda, 2, 2, 70, 2))
+    assert launches == [True]
     assert bool((cache.k_q[:, :, 70:] == 77).all()) and bool((cache.v_q[:, :, 70:] == 77).all())
     assert bool((cache.k_scale[:, :, 3:] == 7).all()) and bool((cache.v_scale[:, :, 70:] == 7).all())
 
 
-def test_rows_the_launch_does_not_take(llmik, cuda):
+def test_rows_the_launch_does_not_take(llmik, cuda, launches):
     """Odd strides and addresses keep the general path's answer: K tokens that
     only fill the open group may have any strides; V may not, nor may either
     be misaligned where a writer reads it."""
@@ -133,6 +151,7 @@ def test_rows_the_launch_does_not_take(llmik, cuda):
     odd = flat[4:].view(v.shape)   # 8 bytes past a 16-byte boundary
     with pytest.raises(RuntimeError):
         kvc.Int4KIVICache(2, 2, 64, 32, device=cuda).append(k, odd)
+    assert launches == [True, False, False, False]
 
 
 def _layer_run(cuda, record):
@@ -146,7 +165,7 @@ def _layer_run(cuda, record):
     return layer, ks, vs, record(layer, ks, vs)
 
 
-def test_gradients_of_the_open_group(llmik, cuda):
+def test_gradients_of_the_open_group(llmik, cuda, launches):
     """The views hold the open group's tokens themselves: their gradient is the
     view's, the quantised tokens' is zero, as through the general path."""
     def record(layer, ks, vs):
@@ -167,6 +186,7 @@ def test_gradients_of_the_open_group(llmik, cuda):
     assert all(t.grad is None or not t.grad.any() for t in (ks[0], vs[0]))
     with torch.no_grad():
         a, b = layer.fp16_view()
+    assert launches and not any(launches[:-1]) and launches[-1]   # the launch again without gradients
     assert not a.requires_grad and torch.equal(a, later[0]) and torch.equal(b, later[1])
 
 
@@ -184,7 +204,7 @@ def test_forward_mode_tangents_of_the_open_group(llmik, cuda):
         assert bool((t[:, :, -21:] == f).all()) and not bool(t[:, :, :-21].any())
 
 
-def test_capture_and_replay(llmik, cuda):
+def test_capture_and_replay(llmik, cuda, launches):
     k, v = _tokens(cuda, 2, 4, 90, 1), _tokens(cuda, 2, 4, 90, 2)
     eager = kvc.Int4KIVICache(2, 4, 128, 32, device=cuda)
     eager.append(k, v)
@@ -194,6 +214,7 @@ def test_capture_and_replay(llmik, cuda):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=s):
         cache.append(k, v)
+    assert launches == [True, True]
     for _ in range(3):
         cache.k_q.zero_()
         cache.v_scale.zero_()
