@@ -177,10 +177,13 @@ static_assert(5 * (kWideGroupLds + sizeof(KScales<kWriterThreads>)) > 160 * 1024
 // is read once. Bound by the read + write stream. With code_words, packed
 // maxima and one reciprocal per channel (us, before -> now): B=8 Hkv=8 S=4096
 // g128 17.5 -> 16.7, g64 16.1 -> 15.5, g32 17.0 -> 15.7; B=64 g32 116 -> 109.
-// Groups of 65-128 tokens are held to 4 workgroups per CU by unused dynamic
-// LDS (kWideGroupLds; the registers would admit 6): B=64 108 -> 105, against
-// 113 with 6, 112 with 5 and 108.8 with 3, as more loads in flight only lengthen the
-// memory queues; B=8 is 2 % slower for it.
+// Groups of 97-128 tokens (7 or 8 real loads a lane) are held to 4 workgroups
+// per CU by unused dynamic LDS (kWideGroupLds; the registers would admit 6)
+// above 128 MiB of input, as more loads in flight then only lengthen the memory
+// queues: g128 B=64 108 -> 105, against 113 with 6, 112 with 5 and 108.8 with 3.
+// us, free -> held, g128 | g112: B=24 S=4096 41.8 -> 40.8 | 42.0 -> 41.3, B=16
+// (128 MiB) 28.8 -> 28.6 | 28.6 -> 28.8, B=8 16.2 -> 16.8 | 16.2 -> 16.7; with
+// fewer real loads it does not pay: g96 B=24 41.2 -> 42.5, g72 42.2 -> 47.6.
 template <int TPR>
 __global__ __launch_bounds__(kWriterThreads) void quantize_k_groupwise_int4_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, uint16_t* __restrict__ scale,
@@ -292,6 +295,8 @@ int launch_quantize_k_groupwise_int4(const void* x, void* q, void* scale, int ro
     auto xp = static_cast<const uint16_t*>(x);
     auto qp = static_cast<int8_t*>(q);
     auto sp = static_cast<uint16_t*>(scale);
+    // Four workgroups per CU (see the kernel).
+    const bool held = group_size > 96 && 256L * n_tok * rows > (128L << 20);
     if (group_size <= 16)
         hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<1>, grid, blk, 0, stream, xp, qp, sp, group_size, map, dst_groups);
     else if (group_size <= 32)
@@ -299,7 +304,7 @@ int launch_quantize_k_groupwise_int4(const void* x, void* q, void* scale, int ro
     else if (group_size <= 64)
         hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<4>, grid, blk, 0, stream, xp, qp, sp, group_size, map, dst_groups);
     else if (group_size <= 128)
-        hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<8>, grid, blk, kWideGroupLds, stream, xp, qp, sp, group_size, map, dst_groups);
+        hipLaunchKernelGGL(quantize_k_groupwise_int4_kernel<8>, grid, blk, held ? kWideGroupLds : 0, stream, xp, qp, sp, group_size, map, dst_groups);
     else
         hipLaunchKernelGGL(quantize_k_groupwise_int4_large_kernel, grid, blk, 0, stream, xp, qp, sp, group_size, map, dst_groups);
     return check_launch();
