@@ -6,6 +6,29 @@
 
 namespace llmik {
 
+// Loads and stores of the elementwise kernels that move each byte once. STREAM
+// (both non-temporal) from kStreamBytes of traffic, what the eight L2s hold
+// together: with plain stores the next kernel also pays for writing the dirty
+// lines back. us, plain -> STREAM: rmsnorm, rope of q and k and silu_mul in
+// turn, T=2000, 32 + 8 heads, 14336 wide 54.2 -> 47.0, T=1000, 11008 wide 29.0
+// -> 25.7, T=4096 97.6 -> 86.7. What reads the output finds less of it in L2:
+// silu_mul and the down projection of [2000, 14336] 255 -> 258, [700, 8192] 50.1
+// -> 51.7, but a layer's prefill without its attention takes the same (T=2000
+// 918 and 920, T=700 305 and 305, T=1000 440 and 441, T=4096 1808 and 1802).
+// Below, the output fits and the reader's loss is all there is: silu_mul and
+// down of [170, 14336] 44.3 -> 45.9, rope [1, 32, 2000, 128] (31 MiB) alone 6.9
+// -> 7.8 and with the K writer 12.5 -> 13.7.
+constexpr long kStreamBytes = 32L << 20;
+template <bool STREAM>
+__device__ __forceinline__ u32x4 ew_load16(const void* p) {
+    return STREAM ? stream16(p) : load16(p);
+}
+template <bool STREAM>
+__device__ __forceinline__ void ew_store16(void* p, u32x4 v) {
+    if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+    else *reinterpret_cast<u32x4*>(p) = v;
+}
+
 // One workgroup per row; 16-byte vectors when the row allows it.
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict__ x,
                                                       const uint16_t* __restrict__ w,
@@ -108,24 +131,21 @@ __global__ __launch_bounds__(256) void rmsnorm_regs_kernel(const uint16_t* __res
 }
 
 
-// Bound by the read + write stream. Plain accesses: non-temporal ones are faster
-// alone ([2000, 14336] 32.6 -> 30.2 us), but the GEMM that reads the output pays
-// for it: with the down projection [170, 14336] 44.3 -> 45.9, [700, 8192] 50.1 ->
-// 51.7, [1500, 8192] 78.5 -> 81.3, [2000, 14336] 255 -> 259; no shape gained.
+template <bool STREAM>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ g,
                                                        const uint16_t* __restrict__ u,
                                                        uint16_t* __restrict__ out, long n) {
     const long i8 = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
     if (i8 + 8 <= n) {
         float gv[8], uv[8];
-        f16x8_to_f32(load16(g + i8), gv);
-        f16x8_to_f32(load16(u + i8), uv);
+        f16x8_to_f32(ew_load16<STREAM>(g + i8), gv);
+        f16x8_to_f32(ew_load16<STREAM>(u + i8), uv);
         u32x4 o;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             o[e] = (uint32_t)f2h_bits(silu_mul1(gv[2 * e], uv[2 * e])) |
                    ((uint32_t)f2h_bits(silu_mul1(gv[2 * e + 1], uv[2 * e + 1])) << 16);
-        *reinterpret_cast<u32x4*>(out + i8) = o;
+        ew_store16<STREAM>(out + i8, o);
     } else {
         for (long i = i8; i < n; ++i) out[i] = f2h_bits(silu_mul1(h2f(g[i]), h2f(u[i])));
     }
@@ -159,10 +179,8 @@ __global__ __launch_bounds__(256) void rope_kernel(const uint16_t* __restrict__ 
 // position's cos and sin are read once for kHeads heads. One thread per pair
 // of values moved 2 bytes per access and read 4 table values for 2 outputs.
 // Bound by the read + write stream; us, before -> now: [1, 32, 2000, 128]
-// 14.0 -> 7.1, [1, 8, 2000, 128] 5.5 -> 3.4, [1, 64, 4096, 128] 64 -> 25. Plain
-// accesses: with non-temporal ones [1, 32, 2000, 128] takes 7.8, and with the K
-// writer that reads it 13.7 against 12.5.
-template <int kHeads>
+// 14.0 -> 7.1, [1, 8, 2000, 128] 5.5 -> 3.4, [1, 64, 4096, 128] 64 -> 24.
+template <int kHeads, bool STREAM>
 __global__ __launch_bounds__(256) void rope_vec_kernel(const uint16_t* __restrict__ x,
                                                        const uint16_t* __restrict__ cs,
                                                        const uint16_t* __restrict__ sn,
@@ -185,8 +203,8 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const uint16_t* __restric
 #pragma unroll
     for (int i = 0; i < kHeads; ++i) {
         const long r = row0 + min(i, H - 1 - h0) * head;
-        x1[i] = load16(x + r);
-        x2[i] = load16(x + r + half_d);
+        x1[i] = ew_load16<STREAM>(x + r);
+        x2[i] = ew_load16<STREAM>(x + r + half_d);
     }
     float c1f[8], c2f[8], s1f[8], s2f[8];
     f16x8_to_f32(c1, c1f);
@@ -210,8 +228,8 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const uint16_t* __restric
             o2[k] = (uint32_t)lo2 | ((uint32_t)hi2 << 16);
         }
         const long r = row0 + i * head;
-        *reinterpret_cast<u32x4*>(out + r) = o1;
-        *reinterpret_cast<u32x4*>(out + r + half_d) = o2;
+        ew_store16<STREAM>(out + r, o1);
+        ew_store16<STREAM>(out + r + half_d, o2);
     }
 }
 
@@ -361,7 +379,8 @@ int launch_rmsnorm(const void* x, const void* w, void* out, int rows, int hidden
 int launch_silu_mul(const void* g, const void* u, void* out, long n, hipStream_t stream) {
     if (n == 0) return LLMIK_OK;
     const long blocks = (n + 256 * 8 - 1) / (256 * 8);
-    hipLaunchKernelGGL(silu_mul_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
+    const auto kernel = 6 * n >= kStreamBytes ? silu_mul_kernel<true> : silu_mul_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
                        static_cast<const uint16_t*>(g), static_cast<const uint16_t*>(u),
                        static_cast<uint16_t*>(out), n);
     return check_launch();
@@ -376,13 +395,15 @@ int launch_rope(const void* x, const void* cs, const void* sn, void* out, int B,
     if (D % 16 == 0 && al16(x) && al16(cs) && al16(sn) && al16(out) && units <= 0x7FFFFFFFL && B <= 65535) {
         // Two heads per thread, or one where that leaves CUs without a
         // workgroup ([1, 64, 4096, 128], heads per thread 1 / 2 / 4 / 8: 24.9,
-        // 24.1, 25.2, 24.2 us, at 2000 tokens and 32 heads 8.3, 8.0, 8.1, 8.3, all
-        // with non-temporal accesses).
+        // 24.1, 25.2, 24.2 us; at 2000 tokens and 32 heads, with non-temporal
+        // accesses, 8.3, 8.0, 8.1, 8.3).
         const unsigned gx = (unsigned)((units + 255) / 256);
         const bool two = H >= 2 && (long)gx * ((H + 1) / 2) * B >= device_cu_count();
         const int ny = two ? (H + 1) / 2 : H;
         if (ny <= 65535) {
-            const auto kernel = two ? rope_vec_kernel<2> : rope_vec_kernel<1>;
+            const bool big = 8 * total >= kStreamBytes;
+            const auto kernel = two ? (big ? rope_vec_kernel<2, true> : rope_vec_kernel<2, false>)
+                                    : (big ? rope_vec_kernel<1, true> : rope_vec_kernel<1, false>);
             hipLaunchKernelGGL(kernel, dim3(gx, ny, B), dim3(256), 0, stream, static_cast<const uint16_t*>(x),
                                static_cast<const uint16_t*>(cs), static_cast<const uint16_t*>(sn),
                                static_cast<uint16_t*>(out), H, S, D, (uint32_t)units);
