@@ -1935,6 +1935,7 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
     L7Words wcur, wnext, wfar;   // stages st, st + 1, st + 2
     load_a(s_a0, st0);
     load_w(wcur, st0);
+    __builtin_amdgcn_sched_barrier(0);   // the wait below counts stage st0 + 1's loads
     load_a(s_a1, st0 + 1);
     load_w(wnext, st0 + 1);
     store_w(wcur, st0);
@@ -2091,10 +2092,10 @@ __global__ __launch_bounds__(kL7Threads) void w4a16_gemm_lds_kernel(GemmParams p
 // barriers run beside the other's MFMAs. Products accumulate per scale group
 // from a zero C operand and are scaled at its end in fp32, as above (same
 // error against 64 bits: f32 output 1.0e-7 at K = 4096, 1.9e-7 at 14336).
-// us, kernel above -> this (M, K, N, group): 2048, 4096, 14336, 128: 260 -> 233
-// (1.03 PFLOP/s; a large fp16 library product reaches 1.31 on this card);
-// 2048, 14336, 4096: 249 -> 224; 2048, 4096, 4096: 74.3 -> 67.9; 512, 4096,
-// 14336: 70.8 -> 63.0; 256, 4096, 14336: 44.8 -> 37.7; 768, 14336, 4096: 122 ->
+// us, kernel above -> this (M, K, N, group): 2048, 4096, 14336, 128: 270 -> 231
+// (1.04 PFLOP/s; a large fp16 library product reaches 1.31 on this card; 231-251
+// by the box); 2048, 14336, 4096: 251 -> 217; 2048, 4096, 4096: 77.0 -> 63.9;
+// 512, 4096, 14336: 73.7 -> 59.6; 256, 4096, 14336: 44.8 -> 37.7; 768, 14336, 4096: 122 ->
 // 103; 600, 11008, 4096: 96.4 -> 78.5; 4096, 4096, 14336: 506 -> 452; group 64,
 // 1000, 4096, 11008: 120 -> 109; group 32, 300, 4096, 14336: 90.7 -> 71.5.
 // Not kept: 256 x 128 tiles of 4 waves (128 x 64 blocks in 16-row strips, the

@@ -1,9 +1,10 @@
-"""CPU: the waits of w4a16_gemm_reg_kernel as compiled into libllmik_hip.so.
+"""CPU: the waits of w4a16_gemm_reg_kernel and w4a16_gemm_lds_kernel as compiled
+into libllmik_hip.so.
 
-The kernel copies activations straight into LDS and waits at the start of each
-stage, with a bare count, for its own copies of two stages ago. The wait is
-right for every order of the loads inside a stage exactly if it leaves at most
-as many vector memory instructions pending as the stage before issued: then
+The kernels copy activations straight into LDS and wait once a stage, with a
+bare count, for the wave's own copies of an earlier stage. The wait is right
+for every order of the loads inside a stage exactly if it leaves at most as
+many vector memory instructions pending as the last stage issued: then
 everything older is complete. Read from the disassembly, whose order the
 source alone does not fix."""
 from __future__ import annotations
@@ -19,6 +20,8 @@ PKG = Path(__file__).resolve().parents[1] / "llm-inference-kernels_amd"
 LIB = PKG / "llmik_cuda" / "libllmik_hip.so"
 OBJDUMP = Path("/opt/rocm/llvm/bin/llvm-objdump")
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+KERNELS = {**{g: rb"_ZN5llmik21w4a16_gemm_reg_kernelILi%dE" % g for g in (32, 64, 128)},
+           "lds": rb"_ZN5llmik21w4a16_gemm_lds_kernelE"}
 
 
 def _device_objects(path):
@@ -36,13 +39,12 @@ def _device_objects(path):
 
 @pytest.fixture(scope="module")
 def listings(tmp_path_factory):
-    """Address, text and branch target of each instruction of the three kernels."""
+    """Address, text and branch target of each instruction of the kernels."""
     if not LIB.exists() or not OBJDUMP.exists():
         pytest.skip("no built library or no llvm-objdump")
     out, d = {}, tmp_path_factory.mktemp("co")
     for k, obj in enumerate(_device_objects(LIB)):
-        names = {g: m.group(0) for g in (32, 64, 128)
-                 if (m := re.search(rb"_ZN5llmik21w4a16_gemm_reg_kernelILi%dE\w+(?=\0)" % g, obj))}
+        names = {g: m.group(0) for g, pat in KERNELS.items() if (m := re.search(pat + rb"\w+(?=\0)", obj))}
         if not names:
             continue
         f = d / f"{k}.o"
@@ -57,15 +59,17 @@ def listings(tmp_path_factory):
                     to = re.search(r"\+0x([0-9a-f]+)>$", ln) if "branch" in m.group(1) else None
                     ins.append((int(m.group(2), 16), m.group(1), base + int(to.group(1), 16) if to else None))
             out[g] = ins
-    assert sorted(out) == [32, 64, 128]
+    assert len(out) == len(KERNELS)
     return out
 
 
 # The prologue's first block: copies, words and scales of the first stage.
-FIRST = {32: 4 + 2 + 2, 64: 4 + 2 + 1, 128: 4 + 2}
+FIRST = {32: 4 + 2 + 2, 64: 4 + 2 + 1, 128: 4 + 2, "lds": 4 + 2 + 2}
+# Unrolled stages and tail; the LDS-staged kernel waits once before its first.
+STAGES = {32: 7, 64: 7, 128: 6, "lds": 4}
 
 
-@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("group", list(KERNELS))
 def test_waits_leave_at_most_the_last_stage_pending(listings, group):
     ins = listings[group]
     at = {a: i for i, (a, _, _) in enumerate(ins)}
@@ -92,5 +96,5 @@ def test_waits_leave_at_most_the_last_stage_pending(listings, group):
                 since[k] = n
                 todo.append(k)
     stages = [w for w in waits.values() if w[0] > 0]
-    assert len(stages) == (6 if group == 128 else 7)
+    assert len(stages) == STAGES[group]
     assert all(left <= issued for left, issued in stages), stages
