@@ -98,7 +98,9 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, Attn
     // leaves a third or more of the CUs idle (129-170 slabs on 256 CUs; below
     // 1280 tokens their extra combine costs more), and above one slab per CU
     // (257-341), where some CUs would do twice the work of others, 3 splits
-    // of 4-wave workgroups even it out. us, H=32 Hkv=8, before -> now, fp16 |
+    // of 4-wave workgroups even it out, as far as their partials fit the static
+    // scratch (slot_cap, for every caller: at 4 heads per workgroup up to 325
+    // slabs; at 8 heads 167-170 slabs take 2 splits and 257-341 none). us, H=32 Hkv=8, before -> now, fp16 |
     // INT8 | INT4 g128:
     //   B=9  S=6000  51 -> 38.5     | 28.3 -> 20.9 | 24.5 -> 16.0
     //   B=12 S=3000  33.5 -> 25.4   | 20.8 -> 15.7 | 19.7 -> 12.9
@@ -162,7 +164,7 @@ AttnPlan plan_attention(int batch, int n_heads, int n_kv_heads, int seqlen, Attn
     if (want > kMaxAttnSplits) want = kMaxAttnSplits;
     if (base_wgs > kMaxCounters) want = 1;   // enough workgroups without splitting
     // Partials stay within the static scratch of the entry point that takes no
-    // workspace (binding with 8 heads per workgroup).
+    // workspace, for the callers that bring one too (one plan, the same bits).
     if (mfma && slot_cap > 0) want = std::min(want, slot_cap);
     if (want < 1) want = 1;
     int chunk = (int)((seqlen + want - 1) / want);

@@ -22,9 +22,9 @@
 
 #include "llmik_internal.hpp"
 
-// 2 MiB: the largest attention workspace on a 256-CU MI355X is ~1.05 MiB
-// (fewer than 2 x CUs split slots of up to 4 heads x 130 fp32, plus the
-// counters); devices with more CUs keep the same margin up to ~480 CUs.
+// 2 MiB: the matrix-core plans keep their partials (split slots of up to 8 heads
+// x 130 fp32, plus the counters) within it, up to the last bytes with 8 heads
+// per workgroup; the VALU plans need ~1.05 MiB on 256 CUs.
 static_assert(LLMIK_NOALLOC_SCRATCH_BYTES == (2u << 20), "scratch size is part of the ABI");
 static __device__ __align__(256) unsigned char scratch[LLMIK_NOALLOC_SCRATCH_BYTES];
 

@@ -276,15 +276,18 @@ _TARGET_LINEAR_NAMES = ("q_proj", "k_proj", "v_proj", "o_proj", "up_proj", "gate
 
 
 def dequant_path_threshold(N: int) -> int:
-    """Rows from which dequantise + matmul (hipBLASLt) beats w4a16_gemm on
-    MI355X, measured at the Llama-3-8B shapes with groups of 256 and more:
-    w4a16_gemm is faster up to 1024 rows for N = 4096 (K = 4096 or 14336;
-    47.1 against 52.6 us and 129.1 against 151.5 at 1024, 70.2 against 64.1
-    at 1536) and up to 768 for N = 14336 (113.2 against 114.3; 139.3 against
-    122.6 at 1024). Groups of 32 to 128 take 0.85-0.92 of those times (233 us
-    at 2048 rows of (4096, 14336), where dequantise + matmul takes 237), so
-    for them the two paths meet near 2048 rows. The reference switches at 256
-    (integration/w4a16_patch.py:89), where w4a16_gemm is 1.8-2.4x faster.
+    """Rows from which dequantise + matmul (hipBLASLt) is taken instead of
+    w4a16_gemm, from both paths' times on one MI355X at the Llama-3-8B shapes
+    (us, w4a16_gemm against dequantise + matmul). With groups of 32, 64 and 256
+    w4a16_gemm is faster up to 1024 rows for N = 4096 (K = 4096 or 14336, group
+    64: 49.4 against 56.7 and 145.8 against 162.5; at 1536 rows 77.3 against
+    67.3 and 253.9 against 209.5) and slower from 1024 for N = 14336 (152.0
+    against 130.1). With groups of 128 the two are within 6 % of each other
+    from here to 2048 rows (N = 14336: 134.6 against 129.6 at 1024, 245.7
+    against 237.5 at 2048; K = 14336, N = 4096: 216.8 against 208.2 at 1536,
+    238.2 against 251.8 at 2048), except K = N = 4096 (72.5 against 81.3 at
+    2048). The reference switches at 256 (integration/w4a16_patch.py:89), where
+    w4a16_gemm is 2.0-2.5x faster.
     Below the threshold the output is also the exact one (fp32 accumulation
     of unrounded weights, within 2e-3 of the float64 product; the fp16
     dequantised weights of the other path are not)."""

@@ -84,7 +84,7 @@ def test_llama_shapes(llmik, cuda, M, K, N):
                                       # 2 <= M <= 16 matrix-core GEMV: 32-column tiles, splits,
                                       # a K range that ends inside a batch
                                       (3, 4096, 96, 128), (16, 1056, 32, 32), (9, 7168, 64, 512),
-                                      # M >= 256 LDS-staged GEMM (256 x 128 tiles, >= 86 of them
+                                      # M >= 256 GEMMs of 256 x 128-tile plans (>= 86 tiles
                                       # on 256 CUs): 2 splits with group 32, one split with group
                                       # 64, 2 splits of whole 256-groups, ragged M with 2 splits
                                       # of 6 and 4 stages, a 256-group cut by the split boundary,
@@ -107,8 +107,9 @@ def test_unaligned_output_pointer(llmik, cuda, M, K, N, f32):
     out; a caller's offset view) takes the per-value stores: same bits as the
     aligned output, nothing written outside it. (128, 4096, 4096) splits K;
     (300, 128, 256) does not. (513, 256, 6144) and (300, 512, 6400) run the
-    LDS-staged GEMM (one store per value, rows past M dropped by the buffer
-    bound), without and with a K split."""
+    register-dequantising GEMM (16- and 8-byte stores at every alignment, rows
+    past M dropped by the buffer bound), without and with a K split; the
+    LDS-staged one is in test_gpu_w4a16_large_groups.py."""
     from llmik_cuda._lib import lib
     q, s, packed = _weights(K, N, 128, 5)
     a = _dev(randn((M, K), 6).astype(np.float16), cuda)
@@ -173,8 +174,9 @@ def test_dequantize_bit_exact(llmik, cuda, K, N, gs):
                                       (2000, 1024, 11008, 64), (768, 1024, 14336, 128),
                                       (2048, 4096, 14336, 128), (3072, 1024, 14336, 32)])
 def test_prefill_sizes_lds_gemm(llmik, cuda, M, K, N, gs):
-    """Prefill sizes on the LDS-staged GEMM (M >= 256 with at least 86
-    256 x 128 tiles), on 256 CUs: (768, 14336, 4096) and (1024, 2048, 4096)
+    """Prefill sizes on the plans of 256 x 128 tiles (M >= 256 with at least 86
+    of them; groups up to 128 run w4a16_gemm_reg_kernel, larger ones
+    w4a16_gemm_lds_kernel, in test_gpu_w4a16_large_groups.py), on 256 CUs: (768, 14336, 4096) and (1024, 2048, 4096)
     with every tile in 2 K splits; (768, 1024, 14336) 256 tiles whole and
     the 80 left in 3 splits of 6, 6 and 4 stages; (2048, 4096, 14336) 768
     whole and 128 in 2; (3072, 1024, 14336) 1280 whole and 64 in 4 (group

@@ -9,7 +9,7 @@ matrix-core kernels take over; any N otherwise). The draws reach the
 both generic fallbacks; the M = 1 matrix-core GEMV and the streaming GEMV
 (weights above 8 MiB) are covered by test_gpu_w4a16.py and
 test_gpu_w4a16_stream.py. A second seeded sweep draws prefill sizes (M
-256-3072, N up to 16384): the LDS-staged GEMM unsplit, with every tile in
+256-3072, N up to 16384): the GEMMs of 256 x 128-tile plans unsplit, with every tile in
 2 K splits and with the tiles past whole rounds split 2 or 4 ways, and the
 64 x 128 and 16-row-tile GEMMs where N or K rule it out. Gate, as in test_gpu_w4a16.py: the fp32-output
 instantiation within 2e-3 of the float64 oracle act @ (q * scale); the
@@ -71,7 +71,7 @@ def test_random_shapes_match_oracle(llmik, cuda, M, K, N, gs, seed):
 
 def _prefill_configs(n: int = 12):
     """Prefill sizes: M 256-3072, K up to 8192 in whole groups (a multiple of
-    64 reaches the LDS-staged GEMM, an odd multiple of 32 the 64 x 128-tile
+    64 reaches the 256 x 128-tile plans, an odd multiple of 32 the 64 x 128-tile
     one), N up to 16384 in multiples of 128 (three draws in four) or 64 (the
     16-row-tile GEMM), group sizes 32-256."""
     rng = np.random.default_rng(20261202)

@@ -1,5 +1,5 @@
 """CPU check of the W4A16 kernels' in-register nibble decodes over every
-byte value: i4x8_to_f16_natural (the LDS-staged GEMM) and
+byte value: i4x8_to_f16_natural (the two GEMMs of 256 x 128-tile plans) and
 i4x8_to_f16_pairs (the 64 x 128-tile GEMM and the GEMVs), both in
 csrc/w4a16.hip.
 
