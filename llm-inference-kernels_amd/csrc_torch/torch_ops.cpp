@@ -396,8 +396,9 @@ py::object kivi_append_int4(const std::optional<Tensor>& k, const std::optional<
         if (t.device() != k_q.device() || (uintptr_t)t.data_ptr() % 16 != 0) return py::none();
     // The open group's tokens pass unchanged into k_open, v_open and the views:
     // where autograd follows them, the general path records that.
-    for (const Tensor& t : all)
-        if ((at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined()) return py::none();
+    const bool grad = at::GradMode::is_enabled();
+    for (const Tensor* t : {&k_open, v_open ? &*v_open : nullptr, k ? &*k : nullptr, v ? &*v : nullptr})
+        if (t && ((grad && t->requires_grad()) || t->_fw_grad(/*level=*/0).defined())) return py::none();
     if (length < 0 || length + n > max_len) return py::none();
     const c10::DeviceGuard guard(k_q.device());
     Tensor kv, vv;
